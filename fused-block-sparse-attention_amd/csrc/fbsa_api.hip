@@ -154,7 +154,8 @@ int fbsa_fwd_rows(const fbsa_attn_desc *d, int64_t i_begin, int64_t i_end, const
 }
 
 size_t fbsa_block_mass_workspace_bytes(const fbsa_attn_desc *d) {
-  return d ? (size_t)(d->B * d->Hq * d->L) * sizeof(float) : 0;
+  if (!d || d->B <= 0 || d->Hkv <= 0 || d->Hq < d->Hkv || d->Hq % d->Hkv || d->nblk <= 0 || d->bs <= 0) return 0;
+  return mass_workspace_bytes(d);
 }
 
 int fbsa_block_mass(const fbsa_attn_desc *d, const void *q, const void *k, float *mass, void *ws, void *stream) {
@@ -167,7 +168,7 @@ int fbsa_block_mass(const fbsa_attn_desc *d, const void *q, const void *k, float
   if (!q || !k || !mass || !ws) return fail(FBSA_EINVAL, "fbsa_block_mass: null pointer");
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(mass, 4) || !aligned(ws, 16))
     return fail(FBSA_EINVAL, "fbsa_block_mass: misaligned pointer");
-  return run_block_mass(d, q, k, mass, (float *)ws, (hipStream_t)stream);
+  return run_block_mass(d, q, k, mass, ws, (hipStream_t)stream);
 }
 
 static int check_pool(const fbsa_pool_desc *d, const void *x, const void *out, const void *out2) {

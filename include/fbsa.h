@@ -98,8 +98,9 @@ int fbsa_fwd_rows(const fbsa_attn_desc *d, int64_t i_begin, int64_t i_end, const
  * Scores are rounded like torch's 16-bit matmul and scale multiply,
  * rnd(rnd(q.k) * scale); the softmax is fp32. Reads d->dtype (bf16 or f16),
  * B, Hq, Hkv, L = nblk * bs, D (64, 128, 256), bs (64, 128), nblk, scale, sq,
- * sk. ws: fbsa_block_mass_workspace_bytes(d) bytes, 16-byte aligned (the row
- * log-sum-exp). Replaces the per-query-block loop of capture_mass. */
+ * sk. ws: fbsa_block_mass_workspace_bytes(d) bytes, 16-byte aligned (each
+ * row's unnormalised sums per key block; at most 1 GiB or 256 query blocks'
+ * worth, longer sequences run in several launches). Replaces the per-query-block loop of capture_mass. */
 size_t fbsa_block_mass_workspace_bytes(const fbsa_attn_desc *d);
 int fbsa_block_mass(const fbsa_attn_desc *d, const void *q, const void *k, float *mass, void *ws, void *stream);
 
