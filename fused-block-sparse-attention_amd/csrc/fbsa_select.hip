@@ -38,7 +38,7 @@ struct PoolArgs {
   int64_t B, H, L, D, bs, nblk, grp, l_valid, Ho;
   int64_t sx[3];
   int op;
-  // optional (mean ops of pool_wave_kernel): the selection's row norm of every
+  // optional (token means): the selection's row norm of every
   // pooled row, at norm[(b * Ho + ho) * norm_pitch + block]; norm_key: rounded
   // up to bf16 (candidate side) instead of fp32 (query side)
   float *norm;
@@ -245,7 +245,10 @@ __global__ __launch_bounds__(256) void pool_kernel(PoolArgs a) {
 // xor-shuffles; only the four wave partials go through LDS. Each lane's loads
 // are issued back to back (fixed trip count; rows past l_valid are read at a
 // clamped address and contribute 0). MEAN_TOK_THEN_GRP gives each wave whole
-// heads; the other ops split the block's tokens over the waves.
+// heads; the other ops split the block's tokens over the waves and, where the
+// blocks alone are few (below), a row wider than 64 elements over workgroups
+// (DC = 8 chunks each, 128 bytes of a 16-bit row; a.D / 64 slices of a block
+// back to back).
 // Workgroups [0, nwg0) pool a0, the rest pool a1 (two tensors in one launch).
 template <typename T, int DC, int BS, int OP>
 __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1, int64_t nwg0) {
@@ -256,18 +259,25 @@ __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane % DC, tl = lane / DC;
   const bool second = (int64_t)blockIdx.x >= nwg0;
   const PoolArgs a = second ? a1 : a0;
-  const int64_t blk = second ? (int64_t)blockIdx.x - nwg0 : (int64_t)blockIdx.x;
-  const int64_t i = blk % a.nblk;
-  const int64_t ho = (blk / a.nblk) % a.Ho;
-  const int64_t b = blk / (a.nblk * a.Ho);
   constexpr int op = OP;
+  // 32-bit index arithmetic (launch indices are below 2^31)
+  uint32_t blk = second ? blockIdx.x - (uint32_t)nwg0 : blockIdx.x;
+  int d0 = 0;  // first element of this workgroup's slice of the row
+  if constexpr (op != FBSA_POOL_MEAN_TOK_THEN_GRP) {
+    const uint32_t ns = (uint32_t)a.D / (8 * DC);
+    d0 = (int)(blk % ns) * (8 * DC);
+    blk /= ns;
+  }
+  const int64_t i = blk % (uint32_t)a.nblk;
+  const int64_t ho = blk / (uint32_t)a.nblk % (uint32_t)a.Ho;
+  const int64_t b = blk / (uint32_t)a.nblk / (uint32_t)a.Ho;
   // valid tokens in the block; 0 for a block wholly past l_valid (never block
   // 0, as l_valid >= 1), whose rows then all read row i * BS - 1 and count as 0
   const int64_t rem = a.l_valid - i * BS;
   const int nval = rem < BS ? (rem > 0 ? (int)rem : 0) : BS;
   auto rowptr = [&](int64_t h, int t) {
     const int tc = t < nval ? t : nval - 1;
-    return (const T *)a.x + b * a.sx[0] + h * a.sx[1] + (i * BS + tc) * a.sx[2] + 8 * c;
+    return (const T *)a.x + b * a.sx[0] + h * a.sx[1] + (i * BS + tc) * a.sx[2] + d0 + 8 * c;
   };
   auto xor_sum = [&](double *v) {
 #pragma unroll
@@ -305,22 +315,39 @@ __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1
       for (int e = 0; e < 8; ++e) r0[e] += (double)round_dt<T>(acc[e] / (double)BS);
     }
   } else if constexpr (op == FBSA_POOL_MEAN_GRP_THEN_TOK) {
-    // tokens split over waves and lanes; per token an exact group sum, rounded mean
-    for (int n = 0; n < RPW; ++n) {
-      const int t = (w + n * NW) * TLW + tl;
-      double g[8];
+    // tokens split over waves and lanes; per token an exact group sum, rounded
+    // mean. A lane's (token, head) rows in order, eight loads in flight.
+    double g[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) g[e] = 0.0;
-#pragma unroll 8
-      for (int64_t hh = 0; hh < a.grp; ++hh) {
-        double v[8];
-        load8<T>(rowptr(ho * a.grp + hh, t), v);
+    for (int e = 0; e < 8; ++e) g[e] = 0.0;
+    const int grp = (int)a.grp, nit = RPW * grp;
+    int ln = 0, lh = 0, n = 0, hh = 0;  // token step and head of the next load, of the next sum
+    for (int q0 = 0; q0 < nit; q0 += 8) {
+      Raw8<T> raw[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) g[e] += v[e];
+      for (int u = 0; u < 8; ++u) {
+        if (q0 + u < nit) raw[u] = load_raw8<T>(rowptr(ho * grp + lh, (w + ln * NW) * TLW + tl));
+        if (++lh == grp) { lh = 0; ++ln; }
       }
-      const bool ok = t < nval && t < BS;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) r0[e] += ok ? (double)round_dt<T>(mean_div(g[e], a.grp)) : 0.0;
+      for (int u = 0; u < 8; ++u)
+        if (q0 + u < nit) {
+          double v[8];
+          decode8<T>(raw[u], v);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) g[e] += v[e];
+          if (++hh == grp) {
+            const int t = (w + n * NW) * TLW + tl;
+            const bool ok = t < nval && t < BS;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              r0[e] += ok ? (double)round_dt<T>(mean_div(g[e], a.grp)) : 0.0;
+              g[e] = 0.0;
+            }
+            hh = 0;
+            ++n;
+          }
+        }
     }
     xor_sum(r0);
   } else {
@@ -362,7 +389,7 @@ __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1
   __syncthreads();
   if (tid < DC * 8) {
     const int cc = tid >> 3, e = tid & 7;
-    const int64_t off = ((b * a.Ho + ho) * a.nblk + i) * a.D + 8 * cc + e;
+    const int64_t off = ((b * a.Ho + ho) * a.nblk + i) * a.D + d0 + 8 * cc + e;
     if (op == FBSA_POOL_MEAN_TOK_THEN_GRP || op == FBSA_POOL_MEAN_GRP_THEN_TOK) {
       double tot = 0.0;
 #pragma unroll
@@ -379,7 +406,7 @@ __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1
       else { ((T *)a.out)[off] = (T)(float)mn; ((T *)a.out2)[off] = (T)(float)mx; }
     }
   }
-  if constexpr (op == FBSA_POOL_MEAN_TOK_THEN_GRP || op == FBSA_POOL_MEAN_GRP_THEN_TOK) {
+  if constexpr (op == FBSA_POOL_MEAN_TOK_THEN_GRP) {
     if (a.norm) {
       // the pooled row's sum of squares over d = 0, 1, ... in order (the sum
       // sel_norms_kernel forms from the stored row)
@@ -526,7 +553,8 @@ __global__ __launch_bounds__(256) void pool_grp_kernel(PoolArgs a, int64_t n) {
   }
 }
 
-template <typename T, int DC, int BS> static void launch_pool_op(const PoolArgs &a, int64_t nwg, hipStream_t s) {
+// SC: 16-byte chunks of a workgroup's slice of the row (token-split ops)
+template <typename T, int DC, int BS, int SC> static void launch_pool_sliced(const PoolArgs &a, int64_t nwg, hipStream_t s) {
   switch (a.op) {
     case FBSA_POOL_MEAN_TOK_THEN_GRP:
       if (a.grp == 1) {
@@ -537,13 +565,26 @@ template <typename T, int DC, int BS> static void launch_pool_op(const PoolArgs 
                          a, nwg);
       return;
     case FBSA_POOL_MEAN_GRP_THEN_TOK:
-      hipLaunchKernelGGL((pool_wave_kernel<T, DC, BS, FBSA_POOL_MEAN_GRP_THEN_TOK>), dim3((unsigned)nwg), dim3(256), 0, s, a,
-                         a, nwg);
+      hipLaunchKernelGGL((pool_wave_kernel<T, SC, BS, FBSA_POOL_MEAN_GRP_THEN_TOK>), dim3((unsigned)(nwg * (DC / SC))),
+                         dim3(256), 0, s, a, a, nwg * (DC / SC));
       return;
     default:  // MAX / MIN / MINMAX share one instantiation (the op picks the outputs)
-      hipLaunchKernelGGL((pool_wave_kernel<T, DC, BS, FBSA_POOL_MINMAX>), dim3((unsigned)nwg), dim3(256), 0, s, a, a, nwg);
+      hipLaunchKernelGGL((pool_wave_kernel<T, SC, BS, FBSA_POOL_MINMAX>), dim3((unsigned)(nwg * (DC / SC))), dim3(256), 0,
+                         s, a, a, nwg * (DC / SC));
       return;
   }
+}
+
+template <typename T, int DC, int BS> static void launch_pool_op(const PoolArgs &a, int64_t nwg, hipStream_t s) {
+  // Slices of 8 chunks while whole-row workgroups are fewer than four per CU, of
+  // 4 (64 bytes of a 16-bit row) while they are fewer than one: a workgroup walks its BS x grp rows in serial steps of eight loads, so few of
+  // them leave the memory idle (group mean of 16 heads over 2, d 256, blocks of
+  // 128: 1999 tokens, 32 blocks, 50 -> 18 us; 16301 tokens, 256 blocks, 82 ->
+  // 39 us). With more, whole rows read better (65536 tokens, 1024 blocks: min /
+  // max 16 us whole, 22 us in slices).
+  if (DC > 4 && nwg < 256) launch_pool_sliced<T, DC, BS, (DC > 4 ? 4 : DC)>(a, nwg, s);
+  else if (DC > 8 && nwg < 1024) launch_pool_sliced<T, DC, BS, (DC > 8 ? 8 : DC)>(a, nwg, s);
+  else launch_pool_sliced<T, DC, BS, DC>(a, nwg, s);
 }
 
 template <typename T, int DC> static bool launch_pool_bs(const PoolArgs &a, int64_t nwg, hipStream_t s) {
