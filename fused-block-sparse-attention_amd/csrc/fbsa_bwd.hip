@@ -543,7 +543,9 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
   // (32-bit division: launch indices are below 2^31)
   uint32_t t = (uint32_t)xcd_remap(blockIdx.x, total);
   const int hin = (int)(t % (uint32_t)a.grp); t /= (uint32_t)a.grp;
-  const int64_t i = t % (uint32_t)a.nblk; t /= (uint32_t)a.nblk;
+  // (dense: the longest walks first)
+  const int64_t i = DENSE ? (uint32_t)a.nblk - 1 - t % (uint32_t)a.nblk : t % (uint32_t)a.nblk;
+  t /= (uint32_t)a.nblk;
   const int hk = (int)(t % (uint32_t)a.Hkv);
   const int64_t b = t / (uint32_t)a.Hkv;
   const int hq = hk * a.grp + hin;
@@ -570,9 +572,16 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
           else valid = inb && j < i;
         } else {
           valid = inb && j <= i && (int64_t)j * BS < a.l_valid;
-          for (int s2 = 0; s2 < s && valid; ++s2) valid = selrow[s2] != j;
           if (valid && (j == i || (int64_t)(j + 1) * BS > a.l_valid)) kind = KIND_ABS;
         }
+      }
+      if (a.mask == FBSA_MASK_TOKEN_CAUSAL) {
+        // a block counts in its first slot only (as in the forward's plan)
+        const int ng = a.kk - s0 < 64 ? (int)(a.kk - s0) : 64;
+        for (int m = 0; m < ng; ++m)
+          if (m < lane && __builtin_amdgcn_readlane(j, m) == j) valid = false;
+        for (int m = 0; m < nout; ++m)
+          if (s_blk[m] == j) valid = false;
       }
       const uint64_t m = __ballot(valid);
       const int pos = nout + __popcll(m & ((1ull << lane) - 1ull));
@@ -641,16 +650,29 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
 
   const T *kbase = (const T *)a.k + b * a.sk[0] + hk * a.sk[1];
   const T *vbase = (const T *)a.v + b * a.sv[0] + hk * a.sv[1];
-  // a per-thread copy plan (offsets computed once, uniform row-0 bases per
-  // chunk); d <= 64 issues through the compiler builtin (four workgroups per
-  // CU, measured faster there than the asm form), d > 64 through the asm form
+  // a per-thread copy plan (offsets computed once, uniform row-0 bases per chunk)
   TilePairPlan<T, C::KC, D, C::NW, C::LPT> plan;
   plan.init(a.sk[2], a.sv[2], w, lane);
-  auto issue = [&](int c) {
-    const int slot = c / C::NCH, ch = c % C::NCH;
-    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(blk_of(slot) * BS + ch * C::KC);
-    plan.template issue<(D <= 64)>(stages + (c % C::NSTAGE) * C::STAGE_BYTES, (const char *)(kbase + row0 * a.sk[2]),
-                                   (const char *)(vbase + row0 * a.sv[2]), w);
+  // list entries read an iteration ahead, as in the forward (with that the asm
+  // copies are the faster form at every head dim: 262144 tokens, d 64, dQ within
+  // a training step 4.01 -> 3.98 ms against copies through the builtin, which
+  // had been faster while each issue waited for its list read)
+  int islot = 0, ich = 0, ist = 0;  // chunk to issue next: slot, place in the slot, stage
+  int slot = 0, ch = 0, cst = 0;    // chunk to compute next
+  int f_iblk, f_kind;
+  float f_gate;
+  auto fetch = [&]() {
+    const int last = nv > 0 ? nv - 1 : 0, si = islot < last ? islot : last, sc = slot < last ? slot : last;
+    f_iblk = blk_of(si);
+    f_kind = kind_of(sc);
+    f_gate = DENSE ? 0.f : s_gate[sc];
+  };
+  auto issue = [&]() {
+    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC;
+    plan.issue(stages + ist * C::STAGE_BYTES, (const char *)(kbase + row0 * a.sk[2]),
+               (const char *)(vbase + row0 * a.sv[2]), w);
+    ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
+    if (++ich == C::NCH) { ich = 0; ++islot; }
   };
 
   // dP^T accumulators start at -delta (16-bit types without the gate gradient, whose
@@ -671,7 +693,11 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
 
 #pragma unroll
   for (int c = 0; c < C::NSTAGE - 1; ++c)
-    if (c < nchunks) issue(c);
+    if (c < nchunks) {
+      fetch();
+      issue();
+    }
+  fetch();
   // the register-operand loads above and the first stages have landed (issued
   // together, so their latencies overlap): the compiler then waits for nothing
   // inside the ring loop, where its own waits would also drain the prefetch
@@ -712,11 +738,12 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
     const int ahead = nchunks - 1 - c;
     wait_ring<C::LPT>(ahead < C::NSTAGE - 2 ? ahead : C::NSTAGE - 2);
     lds_barrier();
-    if (c + C::NSTAGE - 1 < nchunks) issue(c + C::NSTAGE - 1);
+    const int kind = __builtin_amdgcn_readfirstlane(f_kind);
+    const float gt = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f_gate)));
+    if (c + C::NSTAGE - 1 < nchunks) issue();
 
-    const char *Ks = stages + (c % C::NSTAGE) * C::STAGE_BYTES;
+    const char *Ks = stages + cst * C::STAGE_BYTES;
     const char *Vs = Ks + C::TILE_BYTES;
-    const int slot = c / C::NCH, ch = c % C::NCH;
     if (want_dg && ch == 0 && slot > 0 && w == 0) {
       // the previous slot's per-wave sums are in (written before this barrier)
       float v = lane < C::NW ? s_dgw[((slot - 1) & 1) * C::NW + lane] : 0.f;
@@ -724,10 +751,6 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
       for (int x = 1; x < C::NW; x <<= 1) v += shfl_xor_f(v, x);
       if (lane == 0) dgrow[s_raw[slot - 1]] = v;
     }
-    const int kind = kind_of(slot);
-    const float gt = DENSE ? 0.f : s_gate[slot];
-    const int64_t j = blk_of(slot);
-
     f32x4 sacc[C::KC / 16], dpacc[C::KC / 16];
     mm_rows_frag<T, D, C::KC / 16, (D >= 128 ? FBSA_DQ_WIN : 0)>(Ks, qf, sacc, g, p);   // S^T: key 16m+4g+r, query p
     mm_rows_frag<T, D, C::KC / 16, (D >= 128 ? FBSA_DQ_WIN : 0)>(Vs, df, dpacc, g, p,
@@ -746,6 +769,7 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
     // masked keys (key row 16m + r of the chunk valid iff <= lim): a uniform
     // branch, so unmasked chunks (the common case) skip the compares
     if (kind != KIND_FULL) {
+      const int64_t j = blk_of(slot);
       const int64_t lim64 = kind == KIND_DIAG ? (int64_t)tq
                             : kind == KIND_PAD  ? a.l_valid - j * BS - 1
                                                 : ((i - j) * BS + tq < a.l_valid - j * BS - 1 ? (i - j) * BS + tq
@@ -790,6 +814,10 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
       mm_tr_acc<T, D, C::KC, (D >= 128 ? FBSA_BWD_TRWIN : 0), DQSPLIT, 2>(Ks, ds, dqacc, g, p, pp, bacc);
     else
       mm_tr_acc<T, D, C::KC, (D >= 128 ? FBSA_BWD_TRWIN : 0), DQSPLIT>(Ks, ds, dqacc, g, p);
+  
+    cst = cst + 1 == C::NSTAGE ? 0 : cst + 1;
+    if (++ch == C::NCH) { ch = 0; ++slot; }
+    fetch();
   }
 
   // the row's delta as sum P dP (its four lanes' parts); with DINIT dacc holds
@@ -1069,11 +1097,25 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
       // (row < L < 2^31, row strides below 4 GiB: checked by the host)
       const char *qh = qh0, *dh = dh0;
       const float *rh = rh0;
+      // the list entries of the next iteration (the query block it issues, the
+      // entry it computes) are read at the end of this one and go to scalar
+      // registers after its barrier: no LDS read is waited for on the way to an
+      // issue or to the exponentials
+      int cx = 0, cg = 0, cch = 0, cstg = 0;  // chunk to compute next and its stage
+      int f_iq, f_i, f_kind;
+      float f_gate = 0.f;
+      auto fetch = [&]() {
+        f_iq = s_meta[ix < ne ? ix : ne - 1].x;
+        const int c1 = cx < ne ? cx : ne - 1;
+        f_i = s_meta[c1].x;
+        f_kind = s_meta[c1].y;
+        if constexpr (GC) f_gate = __int_as_float(s_meta[c1].z);
+      };
       auto issue = [&]() {
         // uniform: kept in scalar registers, so the tile and row-statistics
         // addresses below are formed by scalar instructions
         const uint32_t row0 =
-            (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)s_meta[ix].x * (uint32_t)BS + (uint32_t)(ic * C::KC)));
+            (uint32_t)__builtin_amdgcn_readfirstlane(f_iq) * (uint32_t)BS + (uint32_t)(ic * C::KC);
         const char *qb = qh + (uint64_t)row0 * qrs;
         const char *db = dh + (uint64_t)row0 * drs;
         char *st = stages + istg * C::STAGE_BYTES;
@@ -1106,9 +1148,12 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
         constexpr int XS = (KEYS / 16) * 64;  // float4 stride between the parts m of a buffer
   #pragma unroll
         for (int c = 0; c < AHEAD; ++c)
-          if (c < nchunks) issue();
+          if (c < nchunks) {
+            fetch();
+            issue();
+          }
+        fetch();
         wait_vmcnt<0>();
-        int cx = 0, cg = 0, cch = 0, cstg = 0;  // chunk c and its stage
         float x[HR / 16][4];                   // pending chunk: P (role 0) or dP (role 1)
         const char *pQ = stages, *pD = stages;
         const float *pM = (const float *)stages;
@@ -1118,6 +1163,9 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
             wait_ring<C::LPT + 1>(ahead < AHEAD - 1 ? ahead : AHEAD - 1);
           }
           lds_barrier();
+          const int kind = __builtin_amdgcn_readfirstlane(f_kind);
+          const float gt = GC ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f_gate))) : 0.f;
+          const int64_t i = __builtin_amdgcn_readfirstlane(f_i);
           if (c + AHEAD < nchunks) issue();
           if (c > 0) {
             if (role == 0) {
@@ -1139,11 +1187,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
           const char *Qs = stages + cstg * C::STAGE_BYTES;
           const char *Ds = Qs + C::TILE_BYTES;
           const float *Ms = (const float *)(Qs + 2 * C::TILE_BYTES);
-          const int4 meta = s_meta[cx];
           const int ch = cch;
-          const int kind = meta.y;
-          const float gt = __int_as_float(meta.z);
-          const int64_t i = meta.x;
           if (++cch == C::NCH) {
             cch = 0;
             if (++cg == a.grp) { cg = 0; ++cx; }
@@ -1183,20 +1227,23 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
               for (int r = 0; r < 4; ++r) x[m][r] = xacc[m][r];
           }
           pQ = Qs; pD = Ds; pM = Ms;
+          fetch();
         }
         continue;
       }
 
   #pragma unroll
       for (int c = 0; c < C::NSTAGE - 1; ++c)
-        if (c < nchunks) issue();
+        if (c < nchunks) {
+          fetch();
+          issue();
+        }
+      fetch();
       // the register-operand loads above and the first stages have landed (issued
       // together, so their latencies overlap): the compiler then waits for nothing
       // inside the ring loop, where its own waits would also drain the prefetch
       wait_vmcnt<0>();
 
-
-      int cx = 0, cg = 0, cch = 0, cstg = 0;  // chunk c and its stage
       if constexpr (dkdv_unrolled<T, BS, D>()) {
         // one role at 16-bit d <= 64: the chunk loop unrolled by the ring depth,
         // each copy reading a fixed stage, so every LDS operand address is a
@@ -1210,12 +1257,11 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
             const int ahead = nchunks - 1 - c;
             wait_ring<C::LPT + 1>(ahead < C::NSTAGE - 2 ? ahead : C::NSTAGE - 2);
             lds_barrier();
+            const int kind = __builtin_amdgcn_readfirstlane(f_kind);
+            const float gt = GC ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f_gate))) : 0.f;
+            const int64_t i = __builtin_amdgcn_readfirstlane(f_i);
             if (c + C::NSTAGE - 1 < nchunks) issue();
-            const int4 meta = s_meta[cx];
             const int ch = cch;
-            const int kind = meta.y;
-            const float gt = __int_as_float(meta.z);
-            const int64_t i = meta.x;
             if (++cch == C::NCH) {
               cch = 0;
               if (++cg == a.grp) { cg = 0; ++cx; }
@@ -1264,6 +1310,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
               mm_tr_acc<T, D, HR, 0, SP, 1, DOFF>(stages, pp, dvacc, g, p);  // dV^T += dO^T P
               mm_tr_acc<T, D, HR, 0, SP, 1, QOFF>(stages, ds, dkacc, g, p);  // dK^T += Q^T dS
             });
+            fetch();
             ++c;
           });
         }
@@ -1276,16 +1323,15 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
         const int ahead = nchunks - 1 - c;
         wait_ring<C::LPT + 1>(ahead < C::NSTAGE - 2 ? ahead : C::NSTAGE - 2);
         lds_barrier();
+        const int kind = __builtin_amdgcn_readfirstlane(f_kind);
+        const float gt = GC ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f_gate))) : 0.f;
+        const int64_t i = __builtin_amdgcn_readfirstlane(f_i);
         if (c + C::NSTAGE - 1 < nchunks) issue();
 
         const char *Qs = stages + cstg * C::STAGE_BYTES;
         const char *Ds = Qs + C::TILE_BYTES;
         const float *Ms = (const float *)(Qs + 2 * C::TILE_BYTES);
-        const int4 meta = s_meta[cx];
         const int ch = cch;
-        const int kind = meta.y;
-        const float gt = __int_as_float(meta.z);
-        const int64_t i = meta.x;
         if (++cch == C::NCH) {
           cch = 0;
           if (++cg == a.grp) { cg = 0; ++cx; }
@@ -1381,6 +1427,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
           tr_acc(SPC, Dh, pp, dvacc);  // dV^T += dO^T P
           tr_acc(SPC, Qh, ds, dkacc);  // dK^T += Q^T dS
         }
+        fetch();
       }
     }
   };

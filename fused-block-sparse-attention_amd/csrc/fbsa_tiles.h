@@ -303,13 +303,11 @@ template <typename T, int KC, int D, int NW, int LPT> struct TilePairPlan {
     }
   }
   // src0 / src1: the first rows of the chunk (wave-uniform)
-  template <bool TRACKED>
   __device__ __forceinline__ void issue(char *st, const char *src0, const char *src1, int w) const {
 #pragma unroll
     for (int n = 0; n < LPT; ++n) {
       const char *base = part[n] ? src1 : src0;
-      if constexpr (TRACKED) g2lds16_tracked(base + off[n], st + (n * NW + w) * 1024);
-      else g2lds16_s(base, off[n], st + (n * NW + w) * 1024);
+      g2lds16_s(base, off[n], st + (n * NW + w) * 1024);
     }
   }
 };
