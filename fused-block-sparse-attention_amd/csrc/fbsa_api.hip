@@ -67,6 +67,12 @@ static int check_attn(const fbsa_attn_desc *d, const char *fn) {
     return fail(FBSA_EINVAL, "%s: L=%lld must equal nblk*bs=%lld", fn, (long long)d->L, (long long)(d->nblk * d->bs));
   if (d->hsel != 1 && d->hsel != d->Hkv) return fail(FBSA_EINVAL, "%s: hsel=%lld must be 1 or Hkv", fn, (long long)d->hsel);
   if (d->l_valid < 1 || d->l_valid > d->L) return fail(FBSA_EINVAL, "%s: l_valid=%lld outside [1, L]", fn, (long long)d->l_valid);
+  if (d->flags & FBSA_FLAG_RAGGED) {
+    if (d->mask == FBSA_MASK_SLOT_CAUSAL)
+      return fail(FBSA_EINVAL, "%s: FBSA_FLAG_RAGGED takes FBSA_MASK_TOKEN_CAUSAL or FBSA_MASK_NONE", fn);
+    if (d->l_valid <= (d->nblk - 1) * d->bs)
+      return fail(FBSA_EINVAL, "%s: FBSA_FLAG_RAGGED needs l_valid=%lld in the last block", fn, (long long)d->l_valid);
+  }
   if (!isfinite(d->scale)) return fail(FBSA_EINVAL, "%s: scale is not finite", fn);
   if (d->B * d->Hq * d->nblk > 0x7fffffffLL) return fail(FBSA_EUNSUPPORTED, "%s: B*Hq*nblk exceeds the grid limit", fn);
   const int64_t es = esize(d->dtype);
@@ -103,6 +109,7 @@ static int check_dense(const fbsa_attn_desc *d, const void *sel, const void *gat
 static void fill_fwd(const fbsa_attn_desc *d, FwdArgs &a) {
   a.B = d->B; a.Hq = d->Hq; a.Hkv = d->Hkv; a.L = d->L; a.nblk = d->nblk; a.kk = d->kk; a.hsel = d->hsel;
   a.l_valid = d->l_valid;
+  a.rows = attn_rows(d);
   for (int x = 0; x < 3; ++x) {
     a.sq[x] = d->sq[x]; a.sk[x] = d->sk[x]; a.sv[x] = d->sv[x]; a.so[x] = d->so[x]; a.sog[x] = d->sog[x];
   }
@@ -136,7 +143,7 @@ int fbsa_fwd_rows(const fbsa_attn_desc *d, int64_t i_begin, int64_t i_end, const
   if (i_begin < 0 || i_end < i_begin || i_end > d->nblk)
     return fail(FBSA_EINVAL, "fbsa_fwd: query-block range [%lld, %lld) outside [0, %lld)", (long long)i_begin,
                 (long long)i_end, (long long)d->nblk);
-  if (d->flags & ~FBSA_FLAG_DENSE) return fail(FBSA_EINVAL, "fbsa_fwd: unknown flags 0x%x", d->flags);
+  if (d->flags & ~(FBSA_FLAG_DENSE | FBSA_FLAG_RAGGED)) return fail(FBSA_EINVAL, "fbsa_fwd: unknown flags 0x%x", d->flags);
   if ((e = check_dense(d, sel, gate, "fbsa_fwd"))) return e;
   if (!q || !k || !v || !o) return fail(FBSA_EINVAL, "fbsa_fwd: null tensor pointer");
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(o, 16))
@@ -326,7 +333,7 @@ namespace fbsa {
 static int check_bwd(const fbsa_attn_desc *d, const char *fn, BwdLayout *lay, const void *ws, size_t ws_bytes) {
   int e = check_attn(d, fn);
   if (e) return e;
-  if (d->flags & ~(FBSA_FLAG_OUT_GATE | FBSA_FLAG_DENSE | FBSA_FLAG_DGATE)) return fail(FBSA_EINVAL, "%s: unknown flags 0x%x", fn, d->flags);
+  if (d->flags & ~(FBSA_FLAG_OUT_GATE | FBSA_FLAG_DENSE | FBSA_FLAG_DGATE | FBSA_FLAG_RAGGED)) return fail(FBSA_EINVAL, "%s: unknown flags 0x%x", fn, d->flags);
   if ((d->flags & FBSA_FLAG_DENSE) && (e = check_dense(d, nullptr, nullptr, fn))) return e;
   e = bwd_layout(d, lay);
   if (e) return e;

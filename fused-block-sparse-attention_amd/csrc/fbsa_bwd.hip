@@ -243,6 +243,7 @@ struct PrepArgs {
   void *dout_attn, *dout_gate;
   int64_t Hq, L, rows;
   int64_t so[3], sdo[3], sog[3];
+  int64_t held;  // rows per head that o, dout and out_gate hold (below L: ragged)
   int og_vec;  // out-gate rows and dout_gate 16-byte aligned: vector loads and stores
 };
 
@@ -294,44 +295,46 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
       const int64_t bh = row / a.L;
       t = row % a.L; h = bh % a.Hq; b = bh / a.Hq;
     }
-    float ov[8], dv[8];
-    load8f<T>((const T *)a.o + b * a.so[0] + h * a.so[1] + t * a.so[2] + 8 * c, ov);
-    load8f<T>((const T *)a.dout + b * a.sdo[0] + h * a.sdo[1] + t * a.sdo[2] + 8 * c, dv);
+    if (t < a.held) {
+      float ov[8], dv[8];
+      load8f<T>((const T *)a.o + b * a.so[0] + h * a.so[1] + t * a.so[2] + 8 * c, ov);
+      load8f<T>((const T *)a.dout + b * a.sdo[0] + h * a.sdo[1] + t * a.sdo[2] + 8 * c, dv);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(ov[e], dv[e], acc);
-    if (a.og) {
-      float gv[8], dav[8], dgv[8];
-      const T *grow = (const T *)a.og + b * a.sog[0] + h * a.sog[1] + t * a.sog[2] + 8 * c;
-      if (a.og_vec) {
-        load8f<T>(grow, gv);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) gv[e] = (float)grow[e];
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float s = 1.f / (1.f + __expf(-gv[e]));
-        dav[e] = dv[e] * s;
-        dgv[e] = dv[e] * ov[e] * (1.f - s);
-      }
-      T *da = (T *)a.dout_attn + row * D + 8 * c;
-      T *dg = (T *)a.dout_gate + row * D + 8 * c;
-      if constexpr (sizeof(T) == 4) {
-        *(f32x4 *)da = f32x4{dav[0], dav[1], dav[2], dav[3]};
-        *(f32x4 *)(da + 4) = f32x4{dav[4], dav[5], dav[6], dav[7]};
-      } else {
-        *(s16x8 *)da = pack8<T>(dav);  // workspace rows: 16-byte aligned
-      }
-      if (a.og_vec) {
-        if constexpr (sizeof(T) == 4) {
-          *(f32x4 *)dg = f32x4{dgv[0], dgv[1], dgv[2], dgv[3]};
-          *(f32x4 *)(dg + 4) = f32x4{dgv[4], dgv[5], dgv[6], dgv[7]};
+      for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(ov[e], dv[e], acc);
+      if (a.og) {
+        float gv[8], dav[8], dgv[8];
+        const T *grow = (const T *)a.og + b * a.sog[0] + h * a.sog[1] + t * a.sog[2] + 8 * c;
+        if (a.og_vec) {
+          load8f<T>(grow, gv);
         } else {
-          *(s16x8 *)dg = pack8<T>(dgv);
-        }
-      } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) dg[e] = (T)dgv[e];
+          for (int e = 0; e < 8; ++e) gv[e] = (float)grow[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float s = 1.f / (1.f + __expf(-gv[e]));
+          dav[e] = dv[e] * s;
+          dgv[e] = dv[e] * ov[e] * (1.f - s);
+        }
+        T *da = (T *)a.dout_attn + row * D + 8 * c;
+        T *dg = (T *)a.dout_gate + ((b * a.Hq + h) * a.held + t) * D + 8 * c;
+        if constexpr (sizeof(T) == 4) {
+          *(f32x4 *)da = f32x4{dav[0], dav[1], dav[2], dav[3]};
+          *(f32x4 *)(da + 4) = f32x4{dav[4], dav[5], dav[6], dav[7]};
+        } else {
+          *(s16x8 *)da = pack8<T>(dav);  // workspace rows: 16-byte aligned
+        }
+        if (a.og_vec) {
+          if constexpr (sizeof(T) == 4) {
+            *(f32x4 *)dg = f32x4{dgv[0], dgv[1], dgv[2], dgv[3]};
+            *(f32x4 *)(dg + 4) = f32x4{dgv[4], dgv[5], dgv[6], dgv[7]};
+          } else {
+            *(s16x8 *)dg = pack8<T>(dgv);
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dg[e] = (T)dgv[e];
+        }
       }
     }
   }
@@ -369,6 +372,7 @@ int run_bwd_prep(const fbsa_attn_desc *d, const BwdLayout &lay, const void *o, c
   a.dout_attn = ws + lay.dout_attn;
   a.dout_gate = dout_gate;
   a.Hq = d->Hq; a.L = d->L; a.rows = d->B * d->Hq * d->L;
+  a.held = attn_rows(d);
   for (int x = 0; x < 3; ++x) { a.so[x] = d->so[x]; a.sdo[x] = d->sdo[x]; a.sog[x] = d->sog[x]; }
   const int64_t es = esize(d->dtype);
   a.og_vec = ((uintptr_t)out_gate % 16 == 0) && ((uintptr_t)dout_gate % 16 == 0) && (d->sog[0] * es) % 16 == 0 &&
@@ -480,6 +484,7 @@ struct BwdArgs {
   float *partials;         // [slot][dK, dV][bs rows][D] fp32
   int64_t seg_entries, seg_entries_xub;  // segment length; bound on extra segments (grid size)
   int64_t B, Hq, Hkv, L, nblk, kk, hsel, l_valid;
+  int64_t rows;  // rows per head that the tensors hold (L, or l_valid when ragged)
   int64_t sq[3], sk[3], sv[3], sdo[3];
   float scale2, scale;
   int mask, grp;
@@ -620,9 +625,12 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
 
   const int tq = w * 16 + p;
   const int64_t qpos = i * BS + tq;
+  // (a row past the tensors' end takes the last one's values; its lse of -inf
+  // makes its P zero, and nothing of it is stored)
+  const int64_t qr = qpos < a.rows ? qpos : a.rows - 1;
   RowFrag<T, D> qf, df;
-  qf.load((const T *)a.q + b * a.sq[0] + hq * a.sq[1] + qpos * a.sq[2], g);
-  df.load((const T *)a.dout + b * a.sdo[0] + hq * a.sdo[1] + qpos * a.sdo[2], g);
+  qf.load((const T *)a.q + b * a.sq[0] + hq * a.sq[1] + qr * a.sq[2], g);
+  df.load((const T *)a.dout + b * a.sdo[0] + hq * a.sdo[1] + qr * a.sdo[2], g);
   // the row statistics: from the prep stage, or (fused) formed here exactly as
   // prep_kernel forms them (below, once the ring's first loads are in flight)
   const bool fused = __is_same(T, bf16) && a.o != nullptr;  // uniform
@@ -630,7 +638,7 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
   float lraw = 0.f;
   float2 rs = make_float2(0.f, 0.f);
   if (fused) {
-    of.load((const T *)a.o + b * a.so[0] + hq * a.so[1] + qpos * a.so[2], g);
+    of.load((const T *)a.o + b * a.so[0] + hq * a.so[1] + qr * a.so[2], g);
     lraw = a.lse[(b * a.Hq + hq) * a.L + qpos];
   } else {
     const int64_t row = (b * a.Hq + hq) * a.L + qpos;
@@ -669,8 +677,11 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
   };
   auto issue = [&]() {
     const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC;
-    plan.issue(stages + ist * C::STAGE_BYTES, (const char *)(kbase + row0 * a.sk[2]),
-               (const char *)(vbase + row0 * a.sv[2]), w);
+    const unsigned st = (unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES;
+    if (row0 + C::KC <= a.rows)
+      plan.issue(st, (const char *)(kbase + row0 * a.sk[2]), (const char *)(vbase + row0 * a.sv[2]), w);
+    else
+      plan.issue_tail(st, (const char *)kbase, (const char *)vbase, a.sk[2] * C::ES, a.sv[2] * C::ES, row0, a.rows, w, lane);
     ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
     if (++ich == C::NCH) { ich = 0; ++islot; }
   };
@@ -837,9 +848,10 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
     }
   }
 
-  T *dqrow = (T *)a.dq + ((b * a.Hq + hq) * a.L + qpos) * D;
+  T *dqrow = (T *)a.dq + ((b * a.Hq + hq) * a.rows + qpos) * D;
 #pragma unroll
   for (int mt = 0; mt < D / 16; ++mt) {
+    if (qpos >= a.rows) break;
     const int d0 = 16 * mt + 4 * g;
     if constexpr (sizeof(T) == 4) {
       *(f32x4 *)(dqrow + d0) = f32x4{dqacc[mt][0] * a.scale, dqacc[mt][1] * a.scale, dqacc[mt][2] * a.scale,
@@ -1019,8 +1031,9 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
   const int role = ROLES == 2 ? (w & 1) : 0, kw = ROLES == 2 ? (w >> 1) : w;
   const int u = kpart * KEYS + kw * 16 + p;  // this lane's key row within block j (B-operand column)
   const int64_t kpos = j * BS + u;
-  const T *krow = (const T *)a.k + b * a.sk[0] + hk * a.sk[1] + kpos * a.sk[2];
-  const T *vrow = (const T *)a.v + b * a.sv[0] + hk * a.sv[1] + kpos * a.sv[2];
+  const int64_t kr = kpos < a.rows ? kpos : a.rows - 1;  // (a key past the tensors' end is masked and not stored)
+  const T *krow = (const T *)a.k + b * a.sk[0] + hk * a.sk[1] + kr * a.sk[2];
+  const T *vrow = (const T *)a.v + b * a.sv[0] + hk * a.sv[1] + kr * a.sv[2];
   RowFrag<T, D> kf, vf;  // two roles: kf holds K (role 0) or V (role 1), vf is unused
   kf.load(ROLES == 2 && role ? vrow : krow, g);
   if constexpr (ROLES == 1) vf.load(vrow, g);
@@ -1118,9 +1131,21 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
             (uint32_t)__builtin_amdgcn_readfirstlane(f_iq) * (uint32_t)BS + (uint32_t)(ic * C::KC);
         const char *qb = qh + (uint64_t)row0 * qrs;
         const char *db = dh + (uint64_t)row0 * drs;
-        char *st = stages + istg * C::STAGE_BYTES;
+        const unsigned st = (unsigned)(uintptr_t)stages + istg * C::STAGE_BYTES;
+        if (row0 + C::KC <= (uint32_t)a.rows) {
   #pragma unroll
-        for (int n = 0; n < C::LPT; ++n) g2lds16_s(tdo[n] ? db : qb, (unsigned)toff[n], st + (n * C::NW + w) * 1024);
+          for (int n = 0; n < C::LPT; ++n) g2lds16_s(tdo[n] ? db : qb, (unsigned)toff[n], st + (n * C::NW + w) * 1024);
+        } else {  // the tensors end within this chunk: its missing rows (P = 0) repeat the last one
+          const int ln = opaque(lane), ws = __builtin_amdgcn_readfirstlane(opaque(w));
+  #pragma unroll 1
+          for (int n = 0; n < C::LPT; ++n) {
+            const bool second = (n * C::NW + ws) * 64 >= C::KC * C::CPR;
+            const int u = (n * C::NW + ws) * 64 + ln - (second ? C::KC * C::CPR : 0);
+            const int row = u / C::CPR, ck = (u % C::CPR) ^ swz(row, C::CPR);
+            const uint32_t r = row0 + row < (uint32_t)a.rows ? row0 + row : (uint32_t)a.rows - 1;
+            g2lds16((second ? dh : qh) + (uint64_t)r * (second ? drs : qrs) + ck * 16, st + (n * C::NW + ws) * 1024);
+          }
+        }
         // wave w copies rows w KC/NW .. (w + 1) KC/NW - 1 of the row statistics (two per lane)
         if (lane < C::KC / (2 * C::NW))
           g2lds16(rh + 2 * (row0 + w * (C::KC / C::NW)) + 4 * lane, st + 2 * C::TILE_BYTES + w * (C::KC / C::NW) * 8);
@@ -1457,8 +1482,9 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
     }
     return;
   }
+  if (kpos >= a.rows) return;
   if constexpr (ROLES == 2) {
-    T *row = (T *)(role ? a.dk : a.dv) + ((b * a.Hkv + hk) * a.L + kpos) * D;
+    T *row = (T *)(role ? a.dk : a.dv) + ((b * a.Hkv + hk) * a.rows + kpos) * D;
     const float sc = role ? a.scale : 1.f;
 #pragma unroll
     for (int mt = 0; mt < D / 16; ++mt) {
@@ -1469,8 +1495,8 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
     }
     return;
   }
-  T *dkrow = (T *)a.dk + ((b * a.Hkv + hk) * a.L + kpos) * D;
-  T *dvrow = (T *)a.dv + ((b * a.Hkv + hk) * a.L + kpos) * D;
+  T *dkrow = (T *)a.dk + ((b * a.Hkv + hk) * a.rows + kpos) * D;
+  T *dvrow = (T *)a.dv + ((b * a.Hkv + hk) * a.rows + kpos) * D;
 #pragma unroll
   for (int mt = 0; mt < D / 16; ++mt) {
     const int d0 = 16 * mt + 4 * g;
@@ -1541,7 +1567,7 @@ __global__ __launch_bounds__(256) void seg_table_kernel(const int32_t *seg_off, 
 template <typename T>
 __global__ __launch_bounds__(256) void dkdv_reduce_kernel(const int32_t *wi_slot, const uint64_t *pos,
                                                           const float *partials, void *dk, void *dv, int64_t nblk,
-                                                          int64_t Hkv, int64_t L, int64_t bs, int64_t D, float scale) {
+                                                          int64_t Hkv, int64_t rows, int64_t bs, int64_t D, float scale) {
   // grid: x = work item, y = a slice of RG * 2048 of its 2 bs D elements (RG
   // 8-element groups per thread, 256 threads), so that a block split into many
   // segments is summed by several workgroups with many loads in flight, while an
@@ -1582,11 +1608,12 @@ __global__ __launch_bounds__(256) void dkdv_reduce_kernel(const int32_t *wi_slot
     if (x >= 2 * n) continue;
     const int which = x >= n;  // 0: dK, 1: dV
     const int64_t e = x - which * n;
+    if (j * bs + e / D >= rows) continue;
     const float sc = which ? 1.f : scale;
     float y[8];
 #pragma unroll
     for (int r = 0; r < 8; ++r) y[r] = acc[gq][r] * sc;
-    T *dst = (T *)(which ? dv : dk) + ((b * Hkv + hk) * L + j * bs) * D + e;  // 16-byte aligned
+    T *dst = (T *)(which ? dv : dk) + ((b * Hkv + hk) * rows + j * bs) * D + e;  // 16-byte aligned
     if constexpr (sizeof(T) == 4) {
       *(f32x4 *)dst = f32x4{y[0], y[1], y[2], y[3]};
       *(f32x4 *)(dst + 4) = f32x4{y[4], y[5], y[6], y[7]};
@@ -1615,6 +1642,7 @@ static void fill_bwd(const fbsa_attn_desc *d, const BwdLayout &lay, char *ws, Bw
   a.seg_entries = a.seg_entries_xub = 0;
   a.B = d->B; a.Hq = d->Hq; a.Hkv = d->Hkv; a.L = d->L; a.nblk = d->nblk; a.kk = d->kk; a.hsel = d->hsel;
   a.l_valid = d->l_valid;
+  a.rows = attn_rows(d);
   for (int x = 0; x < 3; ++x) { a.sq[x] = d->sq[x]; a.sk[x] = d->sk[x]; a.sv[x] = d->sv[x]; a.sdo[x] = d->sdo[x]; }
   if (d->flags & FBSA_FLAG_OUT_GATE) {
     a.dout = ws + lay.dout_attn;
@@ -1768,15 +1796,15 @@ int run_bwd_dkdv(const fbsa_attn_desc *d, const BwdLayout &lay, const void *q, c
   const int32_t *wsl = (const int32_t *)(ws + lay.wi_slot);
   switch (d->dtype) {
     case FBSA_BF16:
-      hipLaunchKernelGGL(dkdv_reduce_kernel<bf16>, g, blk, 0, s, wsl, pos, part, dk, dv, d->nblk, d->Hkv, d->L, d->bs,
+      hipLaunchKernelGGL(dkdv_reduce_kernel<bf16>, g, blk, 0, s, wsl, pos, part, dk, dv, d->nblk, d->Hkv, attn_rows(d), d->bs,
                          d->D, d->scale);
       break;
     case FBSA_F16:
-      hipLaunchKernelGGL(dkdv_reduce_kernel<f16>, g, blk, 0, s, wsl, pos, part, dk, dv, d->nblk, d->Hkv, d->L, d->bs,
+      hipLaunchKernelGGL(dkdv_reduce_kernel<f16>, g, blk, 0, s, wsl, pos, part, dk, dv, d->nblk, d->Hkv, attn_rows(d), d->bs,
                          d->D, d->scale);
       break;
     default:
-      hipLaunchKernelGGL(dkdv_reduce_kernel<float>, g, blk, 0, s, wsl, pos, part, dk, dv, d->nblk, d->Hkv, d->L, d->bs,
+      hipLaunchKernelGGL(dkdv_reduce_kernel<float>, g, blk, 0, s, wsl, pos, part, dk, dv, d->nblk, d->Hkv, attn_rows(d), d->bs,
                          d->D, d->scale);
   }
   return hip_check(hipGetLastError(), "dkdv_reduce_kernel launch");

@@ -64,14 +64,19 @@ __host__ __device__ constexpr int swz(int row, int cpr) {
 // lives in it across the asm.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void g2lds16(const void *gsrc, void *lds_wave_base) {
-  const unsigned m = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_wave_base);
+// The LDS destination is given as a pointer or as its LDS address (the low 32
+// bits of the pointer).
+__device__ __forceinline__ void g2lds16(const void *gsrc, unsigned lds_wave_base) {
+  const unsigned m = __builtin_amdgcn_readfirstlane(lds_wave_base);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(gsrc), "s"(m) : "memory", "m0");
+}
+__device__ __forceinline__ void g2lds16(const void *gsrc, void *lds_wave_base) {
+  g2lds16(gsrc, (unsigned)(uintptr_t)lds_wave_base);
 }
 // The same load with a wave-uniform 64-bit base in SGPRs and a 32-bit per-lane
 // byte offset (the instruction's saddr form): no 64-bit address VALU op per load.
-__device__ __forceinline__ void g2lds16_s(const void *sbase, unsigned voff, void *lds_wave_base) {
-  const unsigned m = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_wave_base);
+__device__ __forceinline__ void g2lds16_s(const void *sbase, unsigned voff, unsigned lds_wave_base) {
+  const unsigned m = __builtin_amdgcn_readfirstlane(lds_wave_base);
   // the base is uniform by contract; readfirstlane puts it in SGPRs (folded away
   // when the compiler already holds it there)
   // (readfirstlane returns int: each half goes through uint32_t so that the
@@ -82,6 +87,16 @@ __device__ __forceinline__ void g2lds16_s(const void *sbase, unsigned voff, void
   const uint64_t sb = ((uint64_t)hi << 32) | (uint64_t)lo;
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(sb), "s"(m)
                : "memory", "m0");
+}
+__device__ __forceinline__ void g2lds16_s(const void *sbase, unsigned voff, void *lds_wave_base) {
+  g2lds16_s(sbase, voff, (unsigned)(uintptr_t)lds_wave_base);
+}
+// x as a value the compiler knows nothing of: what is formed from it stays where
+// it is written (rare branches of a chunk loop, whose per-lane row and column
+// indices would otherwise be formed before the loop and held in registers).
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
 }
 __device__ __forceinline__ void g2lds4(const void *gsrc, void *lds_wave_base) {
   const unsigned m = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_wave_base);

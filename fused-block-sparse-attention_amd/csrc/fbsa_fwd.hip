@@ -175,7 +175,9 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
   float qf32[QT][F32 ? QF : 1];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
-    const T *qrow = (const T *)a.q + b * a.sq[0] + hq * a.sq[1] + (i * BS + tq[qt]) * a.sq[2];
+    // (a row past the tensors' end: the last one's values; its lane stores nothing)
+    const int64_t qr = i * BS + tq[qt] < a.rows ? i * BS + tq[qt] : a.rows - 1;
+    const T *qrow = (const T *)a.q + b * a.sq[0] + hq * a.sq[1] + qr * a.sq[2];
     if constexpr (F32) {
 #pragma unroll
       for (int ks = 0; ks < QF; ++ks) qf32[qt][ks] = ((const float *)qrow)[4 * ks + g];
@@ -233,11 +235,23 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
   auto issue = [&]() {
     const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC;
     const char *kb = kbase + row0 * kstep, *vb = vbase + row0 * vstep;
-    char *st = stages + ist * C::STAGE_BYTES;
+    const unsigned st = (unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES;
+    if (row0 + C::KC <= a.rows) {
 #pragma unroll
-    for (int n = 0; n < C::LPT; ++n) {
-      const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;  // wave-uniform
-      g2lds16_s(part ? vb : kb, (unsigned)doff[n], st + (n * C::NW + w) * 1024);
+      for (int n = 0; n < C::LPT; ++n) {
+        const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;  // wave-uniform
+        g2lds16_s(part ? vb : kb, (unsigned)doff[n], st + (n * C::NW + w) * 1024);
+      }
+    } else {  // the tensors end within this chunk: its missing rows (masked) repeat the last one
+      const int ln = opaque(lane);
+#pragma unroll 1
+      for (int n = 0; n < C::LPT; ++n) {
+        const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;
+        const int u = (n * C::NW + w) * 64 + ln - (part ? C::KC * C::CPR : 0);
+        const int row = u / C::CPR, chunk = (u % C::CPR) ^ swz(row, C::CPR);
+        const int64_t r = row0 + row < a.rows ? row0 + row : a.rows - 1;
+        g2lds16((part ? vbase : kbase) + r * (part ? vstep : kstep) + chunk * 16, st + (n * C::NW + w) * 1024);
+      }
     }
     ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
     if (++ich == C::NCH) { ich = 0; ++islot; }
@@ -494,6 +508,10 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
     float lt = l_run[qt] + shfl_xor_f(l_run[qt], 16);
     lt += shfl_xor_f(lt, 32);
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
+    if (i * BS + tq[qt] >= a.rows) {
+      if (a.lse && g == 0) a.lse[(b * a.Hq + hq) * a.L + i * BS + tq[qt]] = -INFINITY;
+      continue;
+    }
     T *orow = (T *)a.o + b * a.so[0] + hq * a.so[1] + (i * BS + tq[qt]) * a.so[2];
     const T *ogrow = a.og ? (const T *)a.og + b * a.sog[0] + hq * a.sog[1] + (i * BS + tq[qt]) * a.sog[2] : nullptr;
 #pragma unroll

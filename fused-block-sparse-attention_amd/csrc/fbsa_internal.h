@@ -22,7 +22,10 @@ struct FwdArgs {
   int mask;
   int grp;
   int dense;     // FBSA_FLAG_DENSE: slot s is block s, sel and gate unused
+  int64_t rows;  // rows per head that the tensors hold (L, or l_valid with FBSA_FLAG_RAGGED)
 };
+
+inline int64_t attn_rows(const fbsa_attn_desc *d) { return d->flags & FBSA_FLAG_RAGGED ? d->l_valid : d->L; }
 
 // Top-k budgets of fbsa_select: up to kSelListMax on the wave-list kernels,
 // up to kSelWideMax on the row-per-workgroup kernel (its keys live in LDS).

@@ -302,8 +302,23 @@ template <typename T, int KC, int D, int NW, int LPT> struct TilePairPlan {
                           (int64_t)sizeof(T));
     }
   }
-  // src0 / src1: the first rows of the chunk (wave-uniform)
-  __device__ __forceinline__ void issue(char *st, const char *src0, const char *src1, int w) const {
+  // A chunk (from row row0 of the sources at base0 / base1, byte strides step0 /
+  // step1) that runs past the sources' last row: the rows beyond repeat it.
+  __device__ __forceinline__ void issue_tail(unsigned st, const char *base0, const char *base1, int64_t step0, int64_t step1,
+                                             int64_t row0, int64_t rows, int w, int lane) const {
+    constexpr int CPR = D * (int)sizeof(T) / 16;
+    const int ln = opaque(lane), ws = __builtin_amdgcn_readfirstlane(opaque(w));
+#pragma unroll 1
+    for (int n = 0; n < LPT; ++n) {
+      const bool second = (n * NW + ws) * 64 >= KC * CPR;
+      const int u = (n * NW + ws) * 64 + ln - (second ? KC * CPR : 0);
+      const int row = u / CPR, ck = (u % CPR) ^ swz(row, CPR);
+      const int64_t r = row0 + row < rows ? row0 + row : rows - 1;
+      g2lds16((second ? base1 : base0) + r * (second ? step1 : step0) + ck * 16, st + (n * NW + ws) * 1024);
+    }
+  }
+  // st: the stage's LDS address; src0 / src1: the first rows of the chunk (wave-uniform)
+  __device__ __forceinline__ void issue(unsigned st, const char *src0, const char *src1, int w) const {
 #pragma unroll
     for (int n = 0; n < LPT; ++n) {
       const char *base = part[n] ? src1 : src0;

@@ -18,12 +18,12 @@ from . import ops
 
 class BlockSparseAttention(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, k, v, sel, gate, out_gate, mask, scale, l_valid, gate_grad):
+    def forward(ctx, q, k, v, sel, gate, out_gate, mask, scale, l_valid, gate_grad, bs=None):
         o, lse = ops.attention_forward(q, k, v, sel, mask=mask, scale=scale, gate=gate, l_valid=l_valid,
-                                       out_gate=out_gate, need_lse=True)
+                                       out_gate=out_gate, need_lse=True, bs=bs)
         ctx.dense = sel if isinstance(sel, ops.DenseSelection) else None
         ctx.save_for_backward(q, k, v, None if ctx.dense is not None else sel, gate, out_gate, o, lse)
-        ctx.mask, ctx.scale, ctx.l_valid, ctx.gate_grad = mask, scale, l_valid, gate_grad
+        ctx.mask, ctx.scale, ctx.l_valid, ctx.gate_grad, ctx.bs = mask, scale, l_valid, gate_grad, bs
         return o
 
     @staticmethod
@@ -34,17 +34,18 @@ class BlockSparseAttention(torch.autograd.Function):
         need_dg = gate is not None and ctx.gate_grad and ctx.needs_input_grad[4]
         dq, dk, dv, dgate, dog = ops.attention_backward(
             q, k, v, sel, o, lse, do, mask=ctx.mask, scale=ctx.scale, gate=gate, l_valid=ctx.l_valid,
-            out_gate=out_gate, need_dgate=need_dg)
+            out_gate=out_gate, need_dgate=need_dg, bs=ctx.bs)
         if dgate is not None:
             dgate = dgate.to(gate.dtype)
-        return dq, dk, dv, None, dgate, dog, None, None, None, None
+        return dq, dk, dv, None, dgate, dog, None, None, None, None, None
 
 
 def block_sparse_attention(q, k, v, sel, *, mask, scale=None, gate=None, out_gate=None, l_valid=None,
-                           gate_grad=True):
+                           gate_grad=True, bs=None):
     """Differentiable fused block-sparse attention; sel is (B, Hsel, nblk, kk)
-    or an ``ops.DenseSelection`` (every block)."""
-    return BlockSparseAttention.apply(q, k, v, sel, gate, out_gate, mask, scale, l_valid, gate_grad)
+    or an ``ops.DenseSelection`` (every block). bs: block size, given when the
+    last block may be short (``ops.attention_forward``)."""
+    return BlockSparseAttention.apply(q, k, v, sel, gate, out_gate, mask, scale, l_valid, gate_grad, bs)
 
 
 class BSAttnFunction(torch.autograd.Function):

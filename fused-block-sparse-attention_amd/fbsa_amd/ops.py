@@ -74,18 +74,33 @@ def _strides3(t):
     return (t.stride(0), t.stride(1), t.stride(2))
 
 
-def make_desc(q, k, v, o, sel, *, mask, scale, l_valid, dout=None, out_gate=None):
-    B, Hq, L, D = q.shape
+def _block_rows(L, nblk, bs):
+    """Block size and padded length of L rows in nblk blocks: bs None splits L
+    evenly; with bs the last block may be short (its missing rows exist nowhere)."""
+    if nblk == 0 or (bs is None and L % nblk):
+        raise ValueError(f"fbsa: L={L} is not a multiple of nblk={nblk}")
+    if bs is None:
+        return L // nblk, L
+    if not (nblk - 1) * bs < L <= nblk * bs:
+        raise ValueError(f"fbsa: L={L} does not end in the last of {nblk} blocks of {bs}")
+    return bs, nblk * bs
+
+
+def make_desc(q, k, v, o, sel, *, mask, scale, l_valid, dout=None, out_gate=None, bs=None):
+    B, Hq, rows, D = q.shape
     _, hsel, nblk, kk = sel.shape
+    bs, L = _block_rows(rows, nblk, bs)
+    if L != rows and l_valid not in (None, rows):
+        raise ValueError(f"fbsa: l_valid={l_valid} with a short last block of {rows} rows")
     d = _lib.AttnDesc()
     d.dtype = _dtype_code(q)
     d.mask = mask
     d.B, d.Hq, d.Hkv, d.L, d.D = B, Hq, k.shape[1], L, D
-    d.bs = L // nblk
+    d.bs = bs
     d.nblk, d.kk, d.hsel = nblk, kk, hsel
-    d.l_valid = L if l_valid is None else int(l_valid)
+    d.l_valid = rows if l_valid is None else int(l_valid)
     d.scale = float(scale)
-    d.flags = _lib.FLAG_DENSE if isinstance(sel, DenseSelection) else 0
+    d.flags = (_lib.FLAG_DENSE if isinstance(sel, DenseSelection) else 0) | (_lib.FLAG_RAGGED if L != rows else 0)
     d.sq[:] = _strides3(q)
     d.sk[:] = _strides3(k)
     d.sv[:] = _strides3(v)
@@ -113,7 +128,7 @@ def _check_common(q, k, v, sel, gate):
         raise ValueError(f"fbsa: gate shape {tuple(gate.shape)} != sel shape {tuple(sel.shape)}")
 
 
-def prepare_forward(q, k, v, sel, *, mask, scale=None, gate=None, l_valid=None, out_gate=None, need_lse=False):
+def prepare_forward(q, k, v, sel, *, mask, scale=None, gate=None, l_valid=None, out_gate=None, need_lse=False, bs=None):
     """Checks and kernel-ready views for the forward, and its outputs (allocated,
     not yet written). sel must already be the int32 tensor the kernel will read
     (an int32 contiguous sel is used in place, so it may be filled later)."""
@@ -134,10 +149,9 @@ def prepare_forward(q, k, v, sel, *, mask, scale=None, gate=None, l_valid=None, 
     sel32 = sel if dense else sel.to(torch.int32).contiguous()
     gate32 = gate.to(torch.float32).contiguous() if gate is not None else None
     o = torch.empty(B, Hq, L, Dp, dtype=q.dtype, device=q.device)
-    lse = torch.empty(B, Hq, L, dtype=torch.float32, device=q.device) if need_lse else None
-    if sel32.shape[2] == 0 or L % sel32.shape[2]:
-        raise ValueError(f"fbsa: L={L} is not a multiple of nblk={sel32.shape[2]}")
-    d = make_desc(qk[0], qk[1], qk[2], o, sel32, mask=mask, scale=scale, l_valid=l_valid, out_gate=og)
+    Lp = _block_rows(L, sel32.shape[2], bs)[1]
+    lse = torch.empty(B, Hq, Lp, dtype=torch.float32, device=q.device) if need_lse else None
+    d = make_desc(qk[0], qk[1], qk[2], o, sel32, mask=mask, scale=scale, l_valid=l_valid, out_gate=og, bs=bs)
     return {"d": d, "qkv": qk, "sel": None if dense else sel32, "gate": gate32, "og": og, "o": o, "lse": lse,
             "D": D, "Dp": Dp, "nblk": sel32.shape[2]}
 
@@ -160,22 +174,24 @@ def finish_forward(prep, need_lse):
 
 
 def attention_forward(q, k, v, sel, *, mask, scale=None, gate=None, l_valid=None,
-                      out_gate=None, need_lse=False):
+                      out_gate=None, need_lse=False, bs=None):
     """Fused block-sparse attention forward.
 
     q (B,Hq,L,D); k, v (B,Hkv,L,D); sel (B,Hsel,nblk,kk) integer block ids with
     Hsel in {1, Hkv}, or a ``DenseSelection`` (every block, no list); gate (B,Hsel,nblk,kk) additive bias (cast to fp32);
     out_gate (B,Hq,L,D) (any strides): o <- o * sigmoid(out_gate).
-    Returns o (and the fp32 natural-log LSE (B,Hq,L) when need_lse).
+    bs: block size, given when the last of sel's nblk blocks may be short
+    (masks none and token-causal; no padded copies are made).
+    Returns o (and the fp32 natural-log LSE (B,Hq,nblk*bs) when need_lse).
     """
     prep = prepare_forward(q, k, v, sel, mask=mask, scale=scale, gate=gate, l_valid=l_valid, out_gate=out_gate,
-                           need_lse=need_lse)
+                           need_lse=need_lse, bs=bs)
     launch_forward(prep)
     return finish_forward(prep, need_lse)
 
 
 def attention_backward(q, k, v, sel, o, lse, dout, *, mask, scale=None, gate=None, l_valid=None,
-                       out_gate=None, need_dgate=False):
+                       out_gate=None, need_dgate=False, bs=None):
     """Backward of ``attention_forward`` (no atomics; bitwise repeatable).
 
     o and lse are the forward's outputs (o gated when out_gate is given).
@@ -189,8 +205,9 @@ def attention_backward(q, k, v, sel, o, lse, dout, *, mask, scale=None, gate=Non
     B, Hq, L, D = q.shape
     if o.shape != q.shape or dout.shape != q.shape:
         raise ValueError("fbsa: o and dout must have q's shape")
-    if lse.shape != (B, Hq, L) or lse.dtype != torch.float32:
-        raise ValueError("fbsa: lse must be fp32 (B, Hq, L)")
+    Lp = _block_rows(L, sel.shape[2], bs)[1]
+    if lse.shape != (B, Hq, Lp) or lse.dtype != torch.float32:
+        raise ValueError("fbsa: lse must be fp32 (B, Hq, L), L padded to whole blocks")
     scale = D ** -0.5 if scale is None else scale
     Dp = padded_head_dim(D)
     qk = [_kernel_ready(_pad_d(t, Dp)) for t in (q, k, v)]
@@ -207,9 +224,6 @@ def attention_backward(q, k, v, sel, o, lse, dout, *, mask, scale=None, gate=Non
     sel32 = sel if dense else sel.to(torch.int32).contiguous()
     gate32 = gate.to(torch.float32).contiguous() if gate is not None else None
     lse_c = lse.contiguous()
-    nblk = sel32.shape[2]
-    if nblk == 0 or L % nblk:
-        raise ValueError(f"fbsa: L={L} is not a multiple of nblk={nblk}")
     dev = q.device
     dq = torch.empty(B, Hq, L, Dp, dtype=q.dtype, device=dev)
     dk = torch.empty(B, k.shape[1], L, Dp, dtype=q.dtype, device=dev)
@@ -217,7 +231,7 @@ def attention_backward(q, k, v, sel, o, lse, dout, *, mask, scale=None, gate=Non
     dgate = torch.empty(sel32.shape, dtype=torch.float32, device=dev) if need_dgate else None
     dog = torch.empty(B, Hq, L, Dp, dtype=q.dtype, device=dev) if og is not None else None
     d = make_desc(qk[0], qk[1], qk[2], o_p, sel32, mask=mask, scale=scale, l_valid=l_valid, dout=do_p,
-                  out_gate=og)
+                  out_gate=og, bs=bs)
     d.flags |= (_lib.FLAG_OUT_GATE if og is not None else 0) | (_lib.FLAG_DGATE if need_dgate else 0)
     lib = _lib.load()
     nbytes = lib.fbsa_bwd_workspace_bytes(d)

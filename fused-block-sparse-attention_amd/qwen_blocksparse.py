@@ -60,17 +60,13 @@ def blocksparse_forward(q, k, v, *, selector, topk, bs, causal=True, scale=None,
         sel = ops.DenseSelection(B, nblk)
         mask = ops.MASK_TOKEN_CAUSAL if causal else ops.MASK_NONE
     else:
-        idx = selector.select(q, k)
+        idx = _block_list(selector, q, k)
         mask = ops.MASK_TOKEN_CAUSAL
         if tuple(idx.shape[:3]) != (B, Hkv, nblk):
             raise ValueError(f"selector returned {tuple(idx.shape)}, expected ({B}, {Hkv}, {nblk}, kk)")
         sel = idx.to(torch.int32).contiguous()
-    qp, _, pad = _pad_blocks(q, bs)
-    kp, _, _ = _pad_blocks(k, bs)
-    vp, _, _ = _pad_blocks(v, bs)
-    og = _pad_blocks(out_gate, bs)[0] if out_gate is not None else None
-    out = block_sparse_attention(qp, kp, vp, sel, mask=mask, scale=scale, out_gate=og, l_valid=L)
-    return out[..., :L, :] if pad else out
+    # a short last block is handled in the kernels: no padded copies
+    return block_sparse_attention(q, k, v, sel, mask=mask, scale=scale, out_gate=out_gate, bs=bs)
 
 
 def block_mass(q, k, bs, scale=None):
@@ -84,6 +80,18 @@ def block_mass(q, k, bs, scale=None):
     Hkv = k.shape[1]
     m = ops.block_mass(q, k, bs, scale)
     return m.view(B, Hkv, Hq // Hkv, L // bs, L // bs).mean(2)
+
+
+def _block_list(selector, q, k):
+    """selector.select(q, k); for the Quest selectors below without the round
+    trip through int64 (only when the instance's select is the class's own)."""
+    fn = getattr(selector.select, "__func__", None)
+    if fn is not None and selector.select.__self__ is selector:
+        for cls in (SelectMax, SelectLastTok, SelectMaxQMax, SelectTwoStage):
+            if type(selector) is cls and fn is cls.select:
+                with torch.no_grad():
+                    return selector._select32(q, k)
+    return selector.select(q, k)
 
 
 def _finish(score, topk, sink, B, Hkv, nblk, dev):
@@ -113,7 +121,10 @@ class SelectMax:
 
     @torch.no_grad()
     def select(self, q, k):
-        return selection.select_quest(q, k, self.bs, self.topk, sink=self.sink).long()
+        return self._select32(q, k).long()
+
+    def _select32(self, q, k):
+        return selection.select_quest(q, k, self.bs, self.topk, sink=self.sink)
 
 
 class SelectLastTok:
@@ -126,7 +137,10 @@ class SelectLastTok:
 
     @torch.no_grad()
     def select(self, q, k):
-        return selection.select_quest_lasttok(q, k, self.bs, self.topk, sink=self.sink).long()
+        return self._select32(q, k).long()
+
+    def _select32(self, q, k):
+        return selection.select_quest_lasttok(q, k, self.bs, self.topk, sink=self.sink)
 
 
 class SelectMaxQMax:
@@ -142,7 +156,10 @@ class SelectMaxQMax:
 
     @torch.no_grad()
     def select(self, q, k):
-        return selection.select_quest_qmax(q, k, self.bs, self.topk, sink=self.sink).long()
+        return self._select32(q, k).long()
+
+    def _select32(self, q, k):
+        return selection.select_quest_qmax(q, k, self.bs, self.topk, sink=self.sink)
 
 
 class SelectTwoStage:
@@ -155,7 +172,10 @@ class SelectTwoStage:
 
     @torch.no_grad()
     def select(self, q, k):
-        return selection.select_two_stage(q, k, self.bs, self.topk, sink=self.sink, over=self.over).long()
+        return self._select32(q, k).long()
+
+    def _select32(self, q, k):
+        return selection.select_two_stage(q, k, self.bs, self.topk, sink=self.sink, over=self.over)
 
 
 class SelectLearned:

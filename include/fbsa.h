@@ -260,8 +260,14 @@ int fbsa_select_qmax(const fbsa_qmax_desc *d, const void *a, const void *b1, con
  * DGATE (backward): the gate gradient will be asked for (dgate != NULL); the
  * workspace then also holds each query row's probability mass per slot
  * (B*Hq*L*kk fp32), with which a 16-bit gate gradient is corrected to the
- * row's fp32 delta. Required with dgate for 16-bit types. */
-enum { FBSA_FLAG_OUT_GATE = 1, FBSA_FLAG_DENSE = 2, FBSA_FLAG_DGATE = 4 };
+ * row's fp32 delta. Required with dgate for 16-bit types.
+ * RAGGED (forward and backward; NONE and TOKEN_CAUSAL masks): q, k, v, o,
+ * out_gate, dout and every gradient hold l_valid rows per head instead of L
+ * (the last block's rows past l_valid exist nowhere and are neither read nor
+ * written; dq, dk, dv, dout_gate are contiguous over l_valid rows). L is still
+ * nblk * bs, (nblk - 1) * bs < l_valid, and lse keeps L entries per head, -inf
+ * past l_valid. */
+enum { FBSA_FLAG_OUT_GATE = 1, FBSA_FLAG_DENSE = 2, FBSA_FLAG_DGATE = 4, FBSA_FLAG_RAGGED = 8 };
 
 /* Workspace for the backward stages below (one opaque region, 256-byte
  * aligned): per-row softmax statistics, the block-transposed index (CSR of
