@@ -652,6 +652,7 @@ struct SelArgs {
   int64_t ct, nch;                     // MFMA path: candidate tiles per chunk, chunks per row block
   int64_t row0, row1;                  // query blocks (rows) selected by this launch
   int conv, causal, sink, score;
+  int chunked;                         // the caller set the MFMA engine's chunking
 };
 
 // Orderable key: larger = better. Score bits mapped monotonically (NaN above
@@ -694,6 +695,46 @@ __device__ __forceinline__ void list_insert(uint64_t &mine, uint64_t c, int lane
   const uint64_t prev = wave_shr1_u64(mine);
   if (lane > pos && lane < K) mine = prev;
   if (lane == pos) mine = c;
+}
+
+// Writes row i of the selection from its sorted list (lane l: entry l, 0 where
+// there is none): dsc / ssc are the scores of the own block and of block 0.
+__device__ __forceinline__ void sel_write_row(const SelArgs &a, int64_t bh, int64_t i, uint64_t mine, float dsc, float ssc,
+                                              int K, int lane) {
+  const bool convA = a.conv == FBSA_SEL_OWN_FIRST;
+  int32_t *srow = a.sel + (bh * a.nblk + i) * a.kk;
+  float *scrow = a.sel_score ? a.sel_score + (bh * a.nblk + i) * a.kk : nullptr;
+  if (convA) {
+    // slot 0 = own block; slots 1..K = list order; missing picks -> own
+    const uint64_t prev = wave_shr1_u64(mine);
+    if (lane < a.kk) {
+      int idx = (int)i;
+      float sc = dsc;
+      if (lane >= 1 && prev != 0) { idx = key_index(prev); sc = key_score(prev); }
+      srow[lane] = idx;
+      if (scrow) scrow[lane] = sc;
+    }
+  } else {
+    // _finish: K picks (non-finite or missing -> own), own, sink; sorted ascending
+    int idx = (int)i;
+    float sc = dsc;
+    if (lane < K) {
+      if (mine != 0) {
+        const float v = key_score(mine);
+        if (isfinite(v)) { idx = key_index(mine); sc = v; }
+      }
+    } else if (lane == K + 1 && a.sink) { idx = 0; sc = ssc; }
+    const int n = (int)a.kk;
+    int rank = 0;
+    for (int m = 0; m < n; ++m) {
+      const int om = __builtin_amdgcn_readlane(idx, m);
+      rank += (om < idx) || (om == idx && m < lane);
+    }
+    if (lane < n) {
+      srow[rank] = idx;
+      if (scrow) scrow[rank] = sc;
+    }
+  }
 }
 
 template <typename T, int D, int R, int MODE>
@@ -794,41 +835,88 @@ __global__ __launch_bounds__(256) void select_kernel(SelArgs a) {
         if (c == 0) break;
         list_insert(mine, c, lane, K);
       }
-    const float dsc = diag[r];
-    int32_t *srow = a.sel + (bh * a.nblk + i) * a.kk;
-    float *scrow = a.sel_score ? a.sel_score + (bh * a.nblk + i) * a.kk : nullptr;
-    if (convA) {
-      // slot 0 = own block; slots 1..K = list order; missing picks -> own
-      const uint64_t prev = wave_shr1_u64(mine);
-      if (lane < a.kk) {
-        int idx = (int)i;
-        float sc = dsc;
-        if (lane >= 1 && prev != 0) { idx = key_index(prev); sc = key_score(prev); }
-        srow[lane] = idx;
-        if (scrow) scrow[lane] = sc;
-      }
-    } else {
-      // _finish: K picks (non-finite or missing -> own), own, sink; sorted ascending
-      int idx = (int)i;
-      float sc = dsc;
-      if (lane < K) {
-        if (mine != 0) {
-          const float v = key_score(mine);
-          if (isfinite(v)) { idx = key_index(mine); sc = v; }
-        }
-      } else if (lane == K + 1 && a.sink) { idx = 0; sc = sinks[r]; }
-      const int n = (int)a.kk;
-      int rank = 0;
-      for (int m = 0; m < n; ++m) {
-        const int om = __builtin_amdgcn_readlane(idx, m);
-        rank += (om < idx) || (om == idx && m < lane);
-      }
-      if (lane < n) {
-        srow[rank] = idx;
-        if (scrow) scrow[rank] = sc;
+    sel_write_row(a, bh, i, mine, diag[r], sinks[r], K, lane);
+  }
+}
+
+// One wave per query row, for short candidate ranges: lane l scores candidate
+// 64 n + l (the same fp64 sums in the same order as select_kernel), the first 64
+// are ranked against each other by lane reads, later ones inserted. The kernel
+// above gives eight rows to one workgroup, whose first wave inserts the 64
+// candidates of every row one by one: 64 blocks (fp32, d 64) took 38 us on eight
+// workgroups; a wave per row takes 6 us.
+template <typename T, int D, int MODE>
+__global__ __launch_bounds__(256) void select_row_kernel(SelArgs a) {
+  __shared__ __attribute__((aligned(16))) double sa[4][MODE == FBSA_SCORE_QUEST ? 2 : 1][D];
+  __shared__ uint64_t lists[4][64];
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const uint32_t nrows = (uint32_t)(a.row1 - a.row0);
+  const uint32_t rw = blockIdx.x * 4 + w;
+  const bool live = rw < nrows * (uint32_t)(a.B * a.H);
+  const uint32_t rc = live ? rw : 0;
+  const int i = (int)(a.row0 + rc % nrows);
+  const int64_t bh = rc / nrows;
+  const T *A = (const T *)a.a + bh * a.nblk * D;
+  const T *B1 = (const T *)a.b1 + bh * a.nblk * D;
+  const T *B2 = MODE != FBSA_SCORE_DOT ? (const T *)a.b2 + bh * a.nblk * D : nullptr;
+  for (int d = lane; d < D; d += 64) {
+    const double v = (double)(float)A[(int64_t)i * D + d];
+    if constexpr (MODE == FBSA_SCORE_QUEST) { sa[w][0][d] = v > 0.0 ? v : 0.0; sa[w][1][d] = v < 0.0 ? v : 0.0; }
+    else sa[w][0][d] = v;
+  }
+  lists[w][lane] = 0;
+  __syncthreads();
+  if (!live) return;  // wave-uniform; the rest uses no workgroup barrier
+
+  const bool convA = a.conv == FBSA_SEL_OWN_FIRST;
+  const int K = (int)(convA ? (a.topk < a.nblk - 1 ? a.topk : a.nblk - 1) : (a.topk < a.nblk ? a.topk : a.nblk));
+  const int jmax = (a.causal || !convA) ? i : (int)a.nblk - 1;
+  uint64_t mine = 0;
+  float dsc = 0.f, ssc = 0.f;
+  for (int jb = 0; jb <= jmax; jb += 64) {
+    const int j = jb + lane;
+    const bool jin = j <= jmax;
+    const int64_t jr = jin ? j : jmax;
+    double acc = 0.0, acc2 = 0.0;
+#pragma unroll 4
+    for (int d0 = 0; d0 < D; d0 += 8) {
+      double bv[8], bv2[8];
+      load8<T>(B1 + jr * D + d0, bv);
+      if constexpr (MODE != FBSA_SCORE_DOT) load8<T>(B2 + jr * D + d0, bv2);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        acc = __builtin_fma(sa[w][0][d0 + e], bv[e], acc);
+        if constexpr (MODE == FBSA_SCORE_QUEST) acc2 = __builtin_fma(sa[w][1][d0 + e], bv2[e], acc2);
+        else if constexpr (MODE == FBSA_SCORE_MAX2) acc2 = __builtin_fma(sa[w][0][d0 + e], bv2[e], acc2);
       }
     }
+    float sc;
+    if constexpr (MODE == FBSA_SCORE_DOT) sc = round_dt<T>(acc);
+    else if constexpr (MODE == FBSA_SCORE_MAX2) sc = fmaxf(round_dt<T>(acc), round_dt<T>(acc2));
+    else sc = round_dt_f<T>(round_dt<T>(acc) + round_dt<T>(acc2));
+    if (i >= jb && i < jb + 64) dsc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), i - jb));
+    if (jb == 0) ssc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sc), 0));
+    bool cand = jin && K > 0;
+    if (convA) cand = cand && (a.causal ? j < i : j != i);
+    const uint64_t key = cand ? make_key(sc, j) : 0;
+    if (jb == 0) {
+      const int n = jmax < 63 ? jmax + 1 : 64;
+      int rank = 0;
+      for (int m = 0; m < n; ++m) rank += readlane_u64(key, m) > key ? 1 : 0;
+      if (key != 0 && rank < K) lists[w][rank] = key;
+      __builtin_amdgcn_wave_barrier();
+      mine = lists[w][lane];
+      continue;
+    }
+    const uint64_t kth = readlane_u64(mine, K > 0 ? K - 1 : 0);
+    uint64_t surv = __ballot(key > kth);
+    while (surv) {
+      const int src = __ffsll((unsigned long long)surv) - 1;
+      surv &= surv - 1;
+      list_insert(mine, readlane_u64(key, src), lane, K);
+    }
   }
+  sel_write_row(a, bh, i, mine, dsc, ssc, K, lane);
 }
 
 // ------------------------------------------------ wide top-k (K > 62)
@@ -1811,6 +1899,19 @@ static void sel_chunking(int64_t B, int64_t H, int64_t nblk, bool tri, int64_t o
   *nch = (ntiles + c - 1) / c;
 }
 
+// Up to kSelRowMax candidate blocks a wave per row (select_row_kernel) finishes
+// first. Measured (select alone, us, MFMA engine -> row kernel, bf16 d 64): 1 x
+// 64 blocks 29 -> 5, 32 x 32 31 -> 4, 1 x 256 39 -> 11, 16 x 256 39 -> 19; past
+// kSelRowPairs (row, candidate) pairs the MFMA engine is ahead again (64 x 256:
+// 40 -> 51). Against select_kernel (fp32, d 64): 1 x 64 41 -> 6, 1 x 256 55 ->
+// 13, 64 x 256 150 -> 95.
+constexpr int64_t kSelRowMax = 256;
+constexpr int64_t kSelRowPairs = (int64_t)1 << 21;
+static bool sel_row_fits(int conv, int64_t topk, int64_t nblk, int64_t rows, bool mfma) {
+  const int64_t most = conv == FBSA_SEL_OWN_FIRST ? nblk - 1 : nblk, K = topk < most ? topk : most;
+  return nblk <= kSelRowMax && K <= kSelListMax && rows < 0x7fffffffLL && !(mfma && rows * nblk > kSelRowPairs);
+}
+
 // Budgets up to 32: past that the pass-1 bound (the K-th of 64 stream maxima)
 // lets most candidates through and the row buffers are cut over and over
 // (k = 40: 204 against 217 us for the fp64 path over 4096 blocks; k = 48: 759
@@ -1824,7 +1925,13 @@ template <typename T, int D, int MODE> static bool sel_tiled_ok(const SelArgs &a
 
 template <typename T, int D, int MODE> static int launch_sel(const SelArgs &a, void *ws, hipStream_t s) {
   if (a.row1 <= a.row0) return FBSA_OK;
-  if (ws && sel_tiled_ok<T, D, MODE>(a)) {
+  const bool mfma = ws && sel_tiled_ok<T, D, MODE>(a);
+  if (!a.chunked && sel_row_fits(a.conv, a.topk, a.nblk, a.B * a.H * a.nblk, mfma)) {
+    const int64_t nr = a.B * a.H * (a.row1 - a.row0);
+    hipLaunchKernelGGL((select_row_kernel<T, D, MODE>), dim3((unsigned)((nr + 3) / 4)), dim3(256), 0, s, a);
+    return hip_check(hipGetLastError(), "select_row_kernel launch");
+  }
+  if (mfma) {
     if constexpr (sizeof(T) == 2 && (D == 32 || D == 64)) {
       // norms of rows [0, nneed): the query rows' row blocks and every candidate they may select
       const int64_t rb1 = (a.row1 + 63) / 64;
@@ -1918,6 +2025,7 @@ static int run_select_as(const fbsa_select_desc *d, int64_t row0, int64_t row1, 
                (d->flags >> FBSA_SEL_CHUNK_SHIFT) & 0xFFFF, &a.ct, &a.nch);
   a.B = d->B; a.H = d->H; a.nblk = d->nblk; a.D = d->D; a.topk = d->topk; a.kk = d->kk;
   a.conv = d->convention; a.causal = d->causal; a.sink = d->sink; a.score = d->score;
+  a.chunked = ((d->flags >> FBSA_SEL_CHUNK_SHIFT) & 0xFFFF) != 0;
   switch (d->dtype) {
     case FBSA_BF16: return sel_d<bf16>(a, ws, s);
     case FBSA_F16: return sel_d<f16>(a, ws, s);
@@ -1930,12 +2038,12 @@ int run_select(const fbsa_select_desc *d, int64_t row0, int64_t row1, const void
   return run_select_as(d, row0, row1, av, b1, b2, sel, sel_score, ws, 0, s);
 }
 
-// Mean-pooled q.k selection. With the MFMA engine's workspace, 16-bit
-// operands of dim 32 or 64 and a budget of at most 48, q and k are pooled by
-// one launch that also writes the selection's row norms (query side into the
-// first norm array, candidate side into the third; DOT scores use no others),
-// and the selection starts from them; otherwise pool, pool and select run as
-// three calls. Either way qp, kp and sel are the same.
+// Mean-pooled q.k selection. q and k of dim 32 or 64 are pooled by one launch;
+// where the MFMA engine follows (16-bit operands, its workspace, a budget of at
+// most 32, more blocks than select_row_kernel takes) it also writes the
+// selection's row norms (query side into the first norm array, candidate side
+// into the third; DOT scores use no others). Otherwise pool, pool and select run
+// as three calls. Either way qp, kp and sel are the same.
 template <typename T, int D> static int pooled_pair(const fbsa_pool_desc *dq, const void *q, void *qp,
                                                     const fbsa_pool_desc *dk, const void *k, void *kp,
                                                     const fbsa_select_desc *d, float *nq, float *nk, hipStream_t s) {
@@ -1968,21 +2076,31 @@ template <typename T, int D> static int pooled_pair(const fbsa_pool_desc *dq, co
 int run_select_mean_pooled(const fbsa_pool_desc *dq, const void *q, void *qp, const fbsa_pool_desc *dk, const void *k,
                            void *kp, const fbsa_select_desc *d, int32_t *sel, float *sel_score, void *ws, hipStream_t s) {
   const int64_t K = d->topk < d->nblk - 1 ? d->topk : d->nblk - 1;
-  const bool fused = ws && d->dtype != FBSA_F32 && (d->D == 32 || d->D == 64) && K >= 1 && K <= 32 &&
-                     (dq->bs == 16 || dq->bs == 32 || dq->bs == 64 || dq->bs == 128);
-  if (!fused) {
+  const bool pair = (d->D == 32 || d->D == 64) && (dq->bs == 16 || dq->bs == 32 || dq->bs == 64 || dq->bs == 128);
+  const bool norms = pair && ws && d->dtype != FBSA_F32 && K >= 1 && K <= 32 &&
+                     !sel_row_fits(d->convention, d->topk, d->nblk, d->B * d->H * d->nblk, true);
+  if (!pair) {
     int e = run_pool(dq, q, qp, nullptr, s);
     if (!e) e = run_pool(dk, k, kp, nullptr, s);
     return e ? e : run_select(d, 0, d->nblk, qp, kp, nullptr, sel, sel_score, ws, s);
   }
   const int64_t npad = d->B * d->H * sel_norm_pitch(d->nblk);
-  float *nq = (float *)ws, *nk = nq + 2 * npad;
+  float *nq = norms ? (float *)ws : nullptr, *nk = norms ? nq + 2 * npad : nullptr;
   int e;
-  if (d->dtype == FBSA_BF16) e = d->D == 32 ? pooled_pair<bf16, 32>(dq, q, qp, dk, k, kp, d, nq, nk, s)
-                                            : pooled_pair<bf16, 64>(dq, q, qp, dk, k, kp, d, nq, nk, s);
-  else e = d->D == 32 ? pooled_pair<f16, 32>(dq, q, qp, dk, k, kp, d, nq, nk, s)
-                      : pooled_pair<f16, 64>(dq, q, qp, dk, k, kp, d, nq, nk, s);
-  return e ? e : run_select_as(d, 0, d->nblk, qp, kp, nullptr, sel, sel_score, ws, 1, s);
+  switch (d->dtype) {
+    case FBSA_BF16:
+      e = d->D == 32 ? pooled_pair<bf16, 32>(dq, q, qp, dk, k, kp, d, nq, nk, s)
+                     : pooled_pair<bf16, 64>(dq, q, qp, dk, k, kp, d, nq, nk, s);
+      break;
+    case FBSA_F16:
+      e = d->D == 32 ? pooled_pair<f16, 32>(dq, q, qp, dk, k, kp, d, nq, nk, s)
+                     : pooled_pair<f16, 64>(dq, q, qp, dk, k, kp, d, nq, nk, s);
+      break;
+    default:
+      e = d->D == 32 ? pooled_pair<float, 32>(dq, q, qp, dk, k, kp, d, nq, nk, s)
+                     : pooled_pair<float, 64>(dq, q, qp, dk, k, kp, d, nq, nk, s);
+  }
+  return e ? e : run_select_as(d, 0, d->nblk, qp, kp, nullptr, sel, sel_score, ws, norms ? 1 : 0, s);
 }
 
 }  // namespace fbsa
