@@ -754,12 +754,11 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
     f_gate = DENSE ? 0.f : s_gate[sc];
   };
   auto issue = [&]() {
-    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC;
-    const unsigned st = (unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES;
-    if (row0 + C::KC <= a.rows)
-      plan.issue(st, (const char *)(kbase + row0 * a.sk[2]), (const char *)(vbase + row0 * a.sv[2]), w);
-    else
-      plan.issue_tail(st, (const char *)kbase, (const char *)vbase, a.sk[2] * C::ES, a.sv[2] * C::ES, row0, a.rows, w, lane);
+    const uint32_t row0 = tail_row((uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC), (uint32_t)a.rows);
+    plan.issue((unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES, (const char *)(kbase + (int64_t)row0 * a.sk[2]),
+               (const char *)(vbase + (int64_t)row0 * a.sv[2]),
+               tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)(a.sk[2] * C::ES), D * C::ES),
+               tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)(a.sv[2] * C::ES), D * C::ES), w);
     ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
     if (++ich == C::NCH) { ich = 0; ++islot; }
   };
@@ -1207,22 +1206,16 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
         // addresses below are formed by scalar instructions
         const uint32_t row0 =
             (uint32_t)__builtin_amdgcn_readfirstlane(f_iq) * (uint32_t)BS + (uint32_t)(ic * C::KC);
-        const char *qb = qh + (uint64_t)row0 * qrs;
-        const char *db = dh + (uint64_t)row0 * drs;
+        const uint32_t trow = tail_row(row0, (uint32_t)a.rows);
+        const char *qb = qh + (uint64_t)trow * qrs;
+        const char *db = dh + (uint64_t)trow * drs;
         const unsigned st = (unsigned)(uintptr_t)stages + istg * C::STAGE_BYTES;
-        if (row0 + C::KC <= (uint32_t)a.rows) {
+        const uint32_t ql = tail_limit<C::KC>(trow, (uint32_t)a.rows, qrs, D * C::ES);
+        const uint32_t dl = tail_limit<C::KC>(trow, (uint32_t)a.rows, drs, D * C::ES);
   #pragma unroll
-          for (int n = 0; n < C::LPT; ++n) g2lds16_s(tdo[n] ? db : qb, (unsigned)toff[n], st + (n * C::NW + w) * 1024);
-        } else {  // the tensors end within this chunk: its missing rows (P = 0) repeat the last one
-          const int ln = opaque(lane), ws = __builtin_amdgcn_readfirstlane(opaque(w));
-  #pragma unroll 1
-          for (int n = 0; n < C::LPT; ++n) {
-            const bool second = (n * C::NW + ws) * 64 >= C::KC * C::CPR;
-            const int u = (n * C::NW + ws) * 64 + ln - (second ? C::KC * C::CPR : 0);
-            const int row = u / C::CPR, ck = (u % C::CPR) ^ swz(row, C::CPR);
-            const uint32_t r = row0 + row < (uint32_t)a.rows ? row0 + row : (uint32_t)a.rows - 1;
-            g2lds16((second ? dh : qh) + (uint64_t)r * (second ? drs : qrs) + ck * 16, st + (n * C::NW + ws) * 1024);
-          }
+        for (int n = 0; n < C::LPT; ++n) {
+          const uint32_t lim = tdo[n] ? dl : ql;
+          g2lds16_s(tdo[n] ? db : qb, (uint32_t)toff[n] < lim ? (uint32_t)toff[n] : lim, st + (n * C::NW + w) * 1024);
         }
         // wave w copies rows w KC/NW .. (w + 1) KC/NW - 1 of the row statistics (two per lane)
         if (lane < C::KC / (2 * C::NW))

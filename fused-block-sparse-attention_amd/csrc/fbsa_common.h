@@ -91,13 +91,6 @@ __device__ __forceinline__ void g2lds16_s(const void *sbase, unsigned voff, unsi
 __device__ __forceinline__ void g2lds16_s(const void *sbase, unsigned voff, void *lds_wave_base) {
   g2lds16_s(sbase, voff, (unsigned)(uintptr_t)lds_wave_base);
 }
-// x as a value the compiler knows nothing of: what is formed from it stays where
-// it is written (rare branches of a chunk loop, whose per-lane row and column
-// indices would otherwise be formed before the loop and held in registers).
-__device__ __forceinline__ int opaque(int x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
 __device__ __forceinline__ void g2lds4(const void *gsrc, void *lds_wave_base) {
   const unsigned m = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)lds_wave_base);
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(gsrc), "s"(m) : "memory", "m0");

@@ -18,6 +18,7 @@
 
 #include "fbsa_common.h"
 #include "fbsa_internal.h"
+#include "fbsa_tiles.h"
 
 namespace fbsa {
 
@@ -233,25 +234,16 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
     f_gate = DENSE ? 0.f : s_gate[sc];
   };
   auto issue = [&]() {
-    const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC;
-    const char *kb = kbase + row0 * kstep, *vb = vbase + row0 * vstep;
+    const uint32_t row0 = tail_row((uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC), (uint32_t)a.rows);
+    const char *kb = kbase + (int64_t)row0 * kstep, *vb = vbase + (int64_t)row0 * vstep;
+    const uint32_t kl = tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)kstep, D * C::ES);
+    const uint32_t vl = tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)vstep, D * C::ES);
     const unsigned st = (unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES;
-    if (row0 + C::KC <= a.rows) {
 #pragma unroll
-      for (int n = 0; n < C::LPT; ++n) {
-        const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;  // wave-uniform
-        g2lds16_s(part ? vb : kb, (unsigned)doff[n], st + (n * C::NW + w) * 1024);
-      }
-    } else {  // the tensors end within this chunk: its missing rows (masked) repeat the last one
-      const int ln = opaque(lane);
-#pragma unroll 1
-      for (int n = 0; n < C::LPT; ++n) {
-        const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;
-        const int u = (n * C::NW + w) * 64 + ln - (part ? C::KC * C::CPR : 0);
-        const int row = u / C::CPR, chunk = (u % C::CPR) ^ swz(row, C::CPR);
-        const int64_t r = row0 + row < a.rows ? row0 + row : a.rows - 1;
-        g2lds16((part ? vbase : kbase) + r * (part ? vstep : kstep) + chunk * 16, st + (n * C::NW + w) * 1024);
-      }
+    for (int n = 0; n < C::LPT; ++n) {
+      const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;  // wave-uniform
+      const uint32_t lim = part ? vl : kl;
+      g2lds16_s(part ? vb : kb, (uint32_t)doff[n] < lim ? (uint32_t)doff[n] : lim, st + (n * C::NW + w) * 1024);
     }
     ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
     if (++ich == C::NCH) { ich = 0; ++islot; }

@@ -579,8 +579,8 @@ template <typename T, int DC, int BS> static void launch_pool_op(const PoolArgs 
   // Slices of 8 chunks while whole-row workgroups are fewer than four per CU, of
   // 4 (64 bytes of a 16-bit row) while they are fewer than one: a workgroup walks its BS x grp rows in serial steps of eight loads, so few of
   // them leave the memory idle (group mean of 16 heads over 2, d 256, blocks of
-  // 128: 1999 tokens, 32 blocks, 50 -> 18 us; 16301 tokens, 256 blocks, 82 ->
-  // 39 us). With more, whole rows read better (65536 tokens, 1024 blocks: min /
+  // 128: 1999 tokens, 32 blocks, 50 -> 11 us, 18 in slices of 8; 16301 tokens,
+  // 256 blocks, 82 -> 39 us). With more, whole rows read better (65536 tokens, 1024 blocks: min /
   // max 16 us whole, 22 us in slices).
   if (DC > 4 && nwg < 256) launch_pool_sliced<T, DC, BS, (DC > 4 ? 4 : DC)>(a, nwg, s);
   else if (DC > 8 && nwg < 1024) launch_pool_sliced<T, DC, BS, (DC > 8 ? 8 : DC)>(a, nwg, s);

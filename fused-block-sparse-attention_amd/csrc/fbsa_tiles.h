@@ -281,6 +281,19 @@ __device__ __forceinline__ void mm_tr_acc(const char *tile, const float (&x)[KC 
   }
 }
 
+// A chunk of KC rows starting at row0 of a tensor of `rows` rows: the first row
+// to address (row0, or the last row when the chunk lies past the end) and the
+// largest byte offset from it that a copy of the chunk may use. A copy takes its
+// planned offset or, if that is larger, the limit: rows past the end then read
+// the end of the last one (they are masked, or carry P = 0). Whole chunks have
+// no limit. Branch-free, so an issue stays in one basic block with the chunk's
+// reads (as a branch it cost the d 64 kernels 4%).
+__device__ __forceinline__ uint32_t tail_row(uint32_t row0, uint32_t rows) { return row0 < rows ? row0 : rows - 1; }
+template <int KC> __device__ __forceinline__ uint32_t tail_limit(uint32_t row, uint32_t rows, uint32_t step, uint32_t rowbytes) {
+  const uint32_t left = rows - 1 - row;  // row = tail_row(...) < rows
+  return left >= KC - 1 ? 0xffffffffu : left * step + rowbytes - 16;
+}
+
 // Per-thread plan of the direct-to-LDS copy of a KC-row tile pair (two
 // swizzled tiles back to back in one LDS stage, 16-byte loads, LPT per
 // thread): load n reads byte off[n] of source part[n]'s first row (part[n] is
@@ -302,27 +315,14 @@ template <typename T, int KC, int D, int NW, int LPT> struct TilePairPlan {
                           (int64_t)sizeof(T));
     }
   }
-  // A chunk (from row row0 of the sources at base0 / base1, byte strides step0 /
-  // step1) that runs past the sources' last row: the rows beyond repeat it.
-  __device__ __forceinline__ void issue_tail(unsigned st, const char *base0, const char *base1, int64_t step0, int64_t step1,
-                                             int64_t row0, int64_t rows, int w, int lane) const {
-    constexpr int CPR = D * (int)sizeof(T) / 16;
-    const int ln = opaque(lane), ws = __builtin_amdgcn_readfirstlane(opaque(w));
-#pragma unroll 1
-    for (int n = 0; n < LPT; ++n) {
-      const bool second = (n * NW + ws) * 64 >= KC * CPR;
-      const int u = (n * NW + ws) * 64 + ln - (second ? KC * CPR : 0);
-      const int row = u / CPR, ck = (u % CPR) ^ swz(row, CPR);
-      const int64_t r = row0 + row < rows ? row0 + row : rows - 1;
-      g2lds16((second ? base1 : base0) + r * (second ? step1 : step0) + ck * 16, st + (n * NW + ws) * 1024);
-    }
-  }
-  // st: the stage's LDS address; src0 / src1: the first rows of the chunk (wave-uniform)
-  __device__ __forceinline__ void issue(unsigned st, const char *src0, const char *src1, int w) const {
+  // st: the stage's LDS address; src0 / src1: the first rows of the chunk (wave-uniform);
+  // lim0 / lim1: tail_limit of either
+  __device__ __forceinline__ void issue(unsigned st, const char *src0, const char *src1, uint32_t lim0, uint32_t lim1, int w) const {
 #pragma unroll
     for (int n = 0; n < LPT; ++n) {
       const char *base = part[n] ? src1 : src0;
-      g2lds16_s(base, off[n], st + (n * NW + w) * 1024);
+      const uint32_t lim = part[n] ? lim1 : lim0;
+      g2lds16_s(base, off[n] < lim ? off[n] : lim, st + (n * NW + w) * 1024);
     }
   }
 };
