@@ -78,7 +78,8 @@ template <int N> __device__ __forceinline__ void wait_pending(int pending_chunks
   }
 }
 
-template <typename T, int BS, int D, int QT = 1, int KCO = 0, int NSO = 0, bool DENSE = false>
+template <typename T, int BS, int D, int QT = 1, int KCO = 0, int NSO = 0, bool DENSE = false,
+          bool RAGGED = false>
 __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
   using C = FwdCfg<T, BS, D, QT, KCO, NSO>;
   constexpr bool F32 = sizeof(T) == 4;
@@ -177,7 +178,7 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     // (a row past the tensors' end: the last one's values; its lane stores nothing)
-    const int64_t qr = i * BS + tq[qt] < a.rows ? i * BS + tq[qt] : a.rows - 1;
+    const int64_t qr = !RAGGED || i * BS + tq[qt] < a.rows ? i * BS + tq[qt] : a.rows - 1;
     const T *qrow = (const T *)a.q + b * a.sq[0] + hq * a.sq[1] + qr * a.sq[2];
     if constexpr (F32) {
 #pragma unroll
@@ -234,7 +235,8 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
     f_gate = DENSE ? 0.f : s_gate[sc];
   };
   auto issue = [&]() {
-    const uint32_t row0 = tail_row((uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC), (uint32_t)a.rows);
+    const uint32_t first = (uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC);
+    const uint32_t row0 = RAGGED ? tail_row(first, (uint32_t)a.rows) : first;
     const char *kb = kbase + (int64_t)row0 * kstep, *vb = vbase + (int64_t)row0 * vstep;
     const uint32_t kl = tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)kstep, D * C::ES);
     const uint32_t vl = tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)vstep, D * C::ES);
@@ -242,8 +244,8 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
 #pragma unroll
     for (int n = 0; n < C::LPT; ++n) {
       const bool part = (n * C::NW + w) * 64 >= C::KC * C::CPR;  // wave-uniform
-      const uint32_t lim = part ? vl : kl;
-      g2lds16_s(part ? vb : kb, (uint32_t)doff[n] < lim ? (uint32_t)doff[n] : lim, st + (n * C::NW + w) * 1024);
+      const uint32_t lim = part ? vl : kl, off = (uint32_t)doff[n];
+      g2lds16_s(part ? vb : kb, RAGGED && off > lim ? lim : off, st + (n * C::NW + w) * 1024);
     }
     ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
     if (++ich == C::NCH) { ich = 0; ++islot; }
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
     float lt = l_run[qt] + shfl_xor_f(l_run[qt], 16);
     lt += shfl_xor_f(lt, 32);
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
-    if (i * BS + tq[qt] >= a.rows) {
+    if (RAGGED && i * BS + tq[qt] >= a.rows) {
       if (a.lse && g == 0) a.lse[(b * a.Hq + hq) * a.L + i * BS + tq[qt]] = -INFINITY;
       continue;
     }
@@ -535,18 +537,19 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
   }
 }
 
-template <typename T, int BS, int D, int QT = 1, int KCO = 0, int NSO = 0, bool DENSE = false>
+template <typename T, int BS, int D, int QT = 1, int KCO = 0, int NSO = 0, bool DENSE = false,
+          bool RAGGED = false>
 static int launch_fwd_as(const FwdArgs &a, hipStream_t stream) {
   using C = FwdCfg<T, BS, D, QT, KCO, NSO>;
   const size_t lds = (size_t)C::NSTAGE * C::STAGE_BYTES + (DENSE ? 0 : (size_t)a.kk * 12);
   if (lds > 160 * 1024 - 64) return fail(FBSA_EUNSUPPORTED, "fbsa_fwd: kk=%lld needs %zu bytes of LDS", (long long)a.kk, lds);
   {
-    const int e = lds_optin((const void *)fwd_kernel<T, BS, D, QT, KCO, NSO, DENSE>, lds, "hipFuncSetAttribute(fwd)");
+    const int e = lds_optin((const void *)fwd_kernel<T, BS, D, QT, KCO, NSO, DENSE, RAGGED>, lds, "hipFuncSetAttribute(fwd)");
     if (e) return e;
   }
   const int64_t nwg = a.B * a.Hq * a.ni;
   if (nwg == 0) return FBSA_OK;
-  hipLaunchKernelGGL((fwd_kernel<T, BS, D, QT, KCO, NSO, DENSE>), dim3((unsigned)nwg), dim3(C::NT), lds, stream, a);
+  hipLaunchKernelGGL((fwd_kernel<T, BS, D, QT, KCO, NSO, DENSE, RAGGED>), dim3((unsigned)nwg), dim3(C::NT), lds, stream, a);
   return hip_check(hipGetLastError(), "fwd_kernel launch");
 }
 
@@ -554,6 +557,9 @@ static int launch_fwd_as(const FwdArgs &a, hipStream_t stream) {
 // is unchanged by it
 template <typename T, int BS, int D, int QT = 1, int KCO = 0, int NSO = 0>
 static int launch_fwd(const FwdArgs &a, hipStream_t stream) {
+  if (a.rows < a.L)  // short last block: its own instantiation (the limits on its copies cost 1-4%)
+    return a.dense ? launch_fwd_as<T, BS, D, QT, KCO, NSO, true, true>(a, stream)
+                   : launch_fwd_as<T, BS, D, QT, KCO, NSO, false, true>(a, stream);
   return a.dense ? launch_fwd_as<T, BS, D, QT, KCO, NSO, true>(a, stream)
                  : launch_fwd_as<T, BS, D, QT, KCO, NSO, false>(a, stream);
 }
