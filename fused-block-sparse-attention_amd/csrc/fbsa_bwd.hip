@@ -394,20 +394,16 @@ struct IdxArgs {
   int mask;
 };
 
-// Key block of entry e = ((b * hsel + hs) * nblk + i) * kk + slot when the slot
-// is valid under the mask rule, -1 otherwise.
-__device__ __forceinline__ int64_t entry_block(const IdxArgs &a, int64_t e) {
-  const int64_t s = e % a.kk, r = e / a.kk, i = r % a.nblk;
-  const int32_t *row = a.sel + r * a.kk;
-  const int64_t j = row[s];
-  const bool inb = j >= 0 && j < a.nblk;
+// Key block of slot s of selection row r = (b * hsel + hs) * nblk + i when the
+// mask rule lets query block i read it, -1 otherwise (a block chosen twice in a
+// token-causal row is not looked at here: only its first slot counts).
+__device__ __forceinline__ int slot_block(const IdxArgs &a, int64_t r, int64_t i, int64_t s) {
+  const int32_t j = a.sel[r * a.kk + s];
+  if (j < 0 || j >= a.nblk) return -1;
   bool valid;
-  if (a.mask == FBSA_MASK_NONE) valid = inb && j * a.bs < a.l_valid;
-  else if (a.mask == FBSA_MASK_SLOT_CAUSAL) valid = s == 0 ? inb : (inb && j < i);
-  else {
-    valid = inb && j <= i && j * a.bs < a.l_valid;
-    for (int64_t s2 = 0; s2 < s && valid; ++s2) valid = row[s2] != j;
-  }
+  if (a.mask == FBSA_MASK_NONE) valid = j * a.bs < a.l_valid;
+  else if (a.mask == FBSA_MASK_SLOT_CAUSAL) valid = s == 0 || j < i;
+  else valid = j <= i && j * a.bs < a.l_valid;
   return valid ? j : -1;
 }
 
@@ -416,72 +412,131 @@ __device__ __forceinline__ int64_t entry_block(const IdxArgs &a, int64_t e) {
 __global__ __launch_bounds__(256) void keys_kernel(IdxArgs a) {
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= a.n) return;
-  const int64_t j = entry_block(a, e), r = e / a.kk, i = r % a.nblk;
+  const int64_t s = e % a.kk, r = e / a.kk, i = r % a.nblk;
+  int j = slot_block(a, r, i, s);
+  if (a.mask == FBSA_MASK_TOKEN_CAUSAL)
+    for (int64_t s2 = 0; s2 < s && j >= 0; ++s2)
+      if (a.sel[r * a.kk + s2] == j) j = -1;
   a.keys[e] = j >= 0 ? (uint32_t)(r / a.nblk * a.nblk + j) : (uint32_t)a.nseg;
-  a.vals[e] = (int32_t)(i * a.kk + e % a.kk);
+  a.vals[e] = (int32_t)(i * a.kk + s);
 }
 
 // The whole transposed index of a small selection in one launch, one workgroup
-// per (b, hsel): the entries' key blocks in LDS, counted per (part of the
-// entries, key block) by one thread each, offsets by a scan over the blocks, and
-// each thread then writes its entries in order, so a list is ascending as the
-// stable sort leaves it. A group's lists start after the valid entries of the
-// groups before it, which it counts itself. Bound by latency: 8 us for
-// 5120 entries in 32 groups, where the sort's eight launches took 34 us of kernel
-// time (a training step of 32 x 1024 tokens 314 -> 293 us).
-constexpr int kIdxSmallEntries = 16384, kIdxSmallBlocks = 1024;
-__global__ __launch_bounds__(1024) void small_index_kernel(IdxArgs a, int32_t *ent, int32_t *seg_off) {
+// of 16 waves per group (b, hsel): a counting sort of the group's entries by key
+// block, stable, so a list is ascending as the radix sort leaves it.
+// The entries' blocks are staged in LDS. Each wave owns consecutive entries and
+// takes them 64 at a time: lanes with the same block find each other by ballots
+// over its bits, a lane's place among them is a bit count, and the wave's own
+// count per block is one LDS word that the last of them rewrites. The walk runs
+// twice: for the counts, and, once a scan over the waves and blocks has turned
+// these into positions, to place the entries. Its length is the wave's share of
+// the entries whatever the number of blocks. Token-causal rows (a block counts
+// in its first slot only) stay whole within a wave: the word also holds the last
+// row seen, so a repeat is a lane before this one in the same row, or that row.
+// A group's lists start after the valid entries of the groups before it, which
+// it counts as well (repeats in a short row by comparing its slots, in longer
+// ones by the same walk).
+// Bound by the vector instructions of the walk, 1.3 us per 1024 entries and pass.
+constexpr int kIdxWaves = 16;
+constexpr int kIdxShortRow = 8;
+__global__ __launch_bounds__(kIdxWaves * 64) void small_index_kernel(IdxArgs a, int32_t *ent, int32_t *seg_off) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  int *cnt = (int *)smem;                // [parts][NB], 1024 in all
-  int *scan = cnt + 1024;                // [1024]
-  int *red = scan + 1024;                // [16]
-  uint16_t *key = (uint16_t *)(red + 16);  // [nblk * kk]
-  const int tid = threadIdx.x, ng = (int)(a.nblk * a.kk), nblk = (int)a.nblk;
-  const int64_t e0 = (int64_t)blockIdx.x * ng;
-  int NB = 1;
-  while (NB < nblk) NB <<= 1;
-  int before = 0;
-  for (int64_t e = tid; e < e0; e += 1024) before += entry_block(a, e) >= 0 ? 1 : 0;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) before += __shfl_xor(before, m, 64);
-  if ((tid & 63) == 0) red[tid >> 6] = before;
-  for (int e = tid; e < ng; e += 1024) {
-    const int64_t j = entry_block(a, e0 + e);
-    key[e] = j >= 0 ? (uint16_t)j : (uint16_t)0xFFFF;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int nblk = (int)a.nblk, kk = (int)a.kk, ng = nblk * kk, e0 = (int)blockIdx.x * ng, e1 = e0 + ng;
+  const bool token = a.mask == FBSA_MASK_TOKEN_CAUSAL;
+  uint32_t *words = (uint32_t *)smem;              // [kIdxWaves][nblk] (last row + 1) << 16 | count or position
+  int *red = (int *)(words + kIdxWaves * nblk);    // [2][kIdxWaves]
+  uint16_t *key = (uint16_t *)(red + 2 * kIdxWaves);  // [e1]
+  uint32_t *own = words + w * nblk;                // this wave's words
+
+  int before = 0;  // valid entries of earlier groups seen by this wave
+  for (int c = 64 * w; c < e1; c += 64 * kIdxWaves) {
+    const int e = c + lane, r = (uint32_t)e / (uint32_t)kk;
+    const int j = e < e1 ? slot_block(a, r, (uint32_t)r % (uint32_t)nblk, e - r * kk) : -1;
+    if (e < e1) key[e] = (uint16_t)j;  // 0xFFFF: not valid (blocks stay below 1024)
+    if (!token) before += __popcll(__ballot(j >= 0 && e < e0));
   }
+  for (int x = lane; x < nblk; x += 64) own[x] = 0;
+  __syncthreads();
+
+  int bits = 0;
+  while ((1 << bits) < nblk) ++bits;
+  // entries [p0, p1) in order; take(entry, its place in the list of its block), or -1 where it does not count
+  auto walk = [&](int p0, int p1, auto take) {
+    for (int c = p0; c < p1; c += 64) {
+      const int e = c + lane, row = (uint32_t)e / (uint32_t)kk;
+      const int j = e < p1 ? (int)key[e] : 0xFFFF;
+      const bool valid = j != 0xFFFF;
+      uint64_t same = __ballot(valid);
+      for (int x = 0; x < bits; ++x) {
+        const uint64_t one = __ballot((j >> x) & 1);
+        same &= (j >> x) & 1 ? one : ~one;
+      }
+      const uint64_t below = ((uint64_t)1 << lane) - 1;
+      const uint32_t word = valid ? own[j] : 0;
+      bool counts = valid;
+      if (token) {
+        const int first = row * kk - c;  // lane of the row's first slot
+        const uint64_t inrow = first > 0 ? ~(uint64_t)0 << first : ~(uint64_t)0;
+        counts = valid && (int)(word >> 16) != row + 1 && !(same & below & inrow);
+      }
+      const uint64_t mine = __ballot(counts) & same;
+      take(e, counts ? (int)(word & 0xFFFF) + __popcll(mine & below) : -1);
+      if (valid && !(same & ~below & ~((uint64_t)1 << lane)))  // the last lane with this block
+        own[j] = ((uint32_t)(row + 1) << 16) | ((word & 0xFFFF) + (uint32_t)__popcll(mine));
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  if (token && kk <= kIdxShortRow) {
+    for (int c = 64 * w; c < e0; c += 64 * kIdxWaves) {
+      const int e = c + lane;
+      bool counts = e < e0 && key[e] != 0xFFFF;
+      for (int x = (int)((uint32_t)e / (uint32_t)kk) * kk; x < e && counts; ++x) counts = key[x] != key[e];
+      before += __popcll(__ballot(counts));
+    }
+  } else if (token && e0) {
+    const int len = (int)((blockIdx.x * nblk + kIdxWaves - 1) / kIdxWaves) * kk, p0 = w * len < e0 ? w * len : e0;
+    walk(p0, p0 + len < e0 ? p0 + len : e0, [&](int, int at) { before += __popcll(__ballot(at >= 0)); });
+    for (int x = lane; x < nblk; x += 64) own[x] = 0;
+  }
+  const int unit = token ? kk : 1, len = (ng / unit + kIdxWaves - 1) / kIdxWaves * unit;
+  const int p0 = e0 + (w * len < ng ? w * len : ng), p1 = p0 + len < e1 ? p0 + len : e1;
+  walk(p0, p1, [](int, int) {});
+  if (lane == 0) red[w] = before;
+  __syncthreads();
+
+  // thread j: block j's list over the waves, then its first position
+  int tot = 0;
+  if (tid < nblk)
+    for (int x = 0; x < kIdxWaves; ++x) tot += (int)(words[x * nblk + tid] & 0xFFFF);
+  int upto = tot;
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) {
+    const int v = __shfl_up(upto, m, 64);
+    if (lane >= m) upto += v;
+  }
+  if (lane == 63) red[kIdxWaves + w] = upto;
   __syncthreads();
   int base = 0;
 #pragma unroll
-  for (int x = 0; x < 16; ++x) base += red[x];
-  const int parts = 1024 / NB, j = tid & (NB - 1), part = tid / NB, len = (ng + parts - 1) / parts;
-  const int p0 = part * len < ng ? part * len : ng, p1 = p0 + len < ng ? p0 + len : ng;
-  int c = 0;
-  for (int e = p0; e < p1; ++e) c += key[e] == j ? 1 : 0;
-  cnt[tid] = c;
-  __syncthreads();
-  int tot = 0;
-  if (tid < NB)
-    for (int x = 0; x < parts; ++x) {  // exclusive counts over the parts
-      const int v = cnt[x * NB + tid];
-      cnt[x * NB + tid] = tot;
-      tot += v;
+  for (int x = 0; x < kIdxWaves; ++x) {
+    base += red[x];
+    if (x < w) upto += red[kIdxWaves + x];
+  }
+  if (tid < nblk) {
+    int pos = upto - tot;
+    seg_off[(int64_t)blockIdx.x * nblk + tid] = base + pos;
+    if (tid == nblk - 1 && blockIdx.x == gridDim.x - 1) seg_off[a.nseg] = base + upto;
+    for (int x = 0; x < kIdxWaves; ++x) {
+      const int v = (int)(words[x * nblk + tid] & 0xFFFF);
+      words[x * nblk + tid] = (uint32_t)pos;  // (no row: the second walk sees every row anew)
+      pos += v;
     }
-  scan[tid] = tot;  // 0 past NB
-  for (int off = 1; off < NB; off <<= 1) {  // inclusive scan over the blocks
-    __syncthreads();
-    const int v = tid >= off ? scan[tid - off] : 0;
-    __syncthreads();
-    scan[tid] += v;
   }
   __syncthreads();
-  const int first = base + (j ? scan[j - 1] : 0);
-  if (part == 0 && j < nblk) {
-    seg_off[(int64_t)blockIdx.x * nblk + j] = first;
-    if (j == nblk - 1 && blockIdx.x == gridDim.x - 1) seg_off[a.nseg] = base + scan[j];
-  }
-  int pos = first + cnt[tid];
-  for (int e = p0; e < p1; ++e)
-    if (key[e] == j) ent[pos++] = e;
+  walk(p0, p1, [&](int e, int at) {
+    if (at >= 0) ent[base + at] = e - e0;
+  });
 }
 
 // seg_off[x] = first sorted position whose key is >= x, for x in [0, nseg].
@@ -506,6 +561,25 @@ __global__ __launch_bounds__(256) void dense_seg_off_kernel(int32_t *seg_off, in
   seg_off[x] = (int32_t)(grp * dense_prefix(nblk, nblk, nkb, causal) + dense_prefix(j, nblk, nkb, causal));
 }
 
+// The one-launch index, where it is ahead of the sort (whose launches take 11 us
+// up to 1024 entries, 20 us at 2304 and 30 to 33 us from 4096 on): its staged
+// entries and words fit the LDS (16384 entries, 1024 blocks), no CU gets more
+// than two of its workgroups, and its longest walk, twice over a group's own
+// entries and once over the earlier ones of longer token-causal rows, stays
+// within kIdxWalk.
+// Measured (the index stage alone, us, this kernel / the sort; slot-causal and
+// token-causal where they differ): 1 group x 32 blocks x 5 slots 5 / 11, 32 x 32 x
+// 5 7 and 10 / 30, 1 x 128 x 18 9 / 20, 2 x 128 x 18 10 and 13 / 31, 7 x 128 x 18
+// 15 and 27 / 31, 1 x 512 x 16 22 / 31, 16 x 1024 x 1 14 and 17 / 31, 512 x 8 x 4
+// 17 and 24 / 31. Past the line: 1 x 1024 x 16 44 / 31, 2 x 512 x 16 (token-causal)
+// 34 / 32, 1024 x 4 x 4 26 and 40 / 31.
+constexpr int64_t kIdxEntries = 16384, kIdxBlocks = 1024, kIdxGroups = 512, kIdxWalk = 18432;
+static bool small_index_fits(const fbsa_attn_desc *d, int64_t n) {
+  const int64_t own = d->nblk * d->kk;
+  const int64_t earlier = d->mask == FBSA_MASK_TOKEN_CAUSAL && d->kk > kIdxShortRow ? n - own : 0;
+  return n <= kIdxEntries && d->nblk <= kIdxBlocks && d->B * d->hsel <= kIdxGroups && 2 * own + earlier <= kIdxWalk;
+}
+
 int run_transpose_index(const fbsa_attn_desc *d, const BwdLayout &lay, const int32_t *sel, char *ws, hipStream_t s) {
   if (d->flags & FBSA_FLAG_DENSE) {
     const int64_t nkb = (d->l_valid + d->bs - 1) / d->bs;
@@ -520,10 +594,11 @@ int run_transpose_index(const fbsa_attn_desc *d, const BwdLayout &lay, const int
   a.vals = (int32_t *)(ws + lay.vals_in);
   a.nblk = d->nblk; a.kk = d->kk; a.n = lay.n; a.nseg = lay.nseg; a.bs = d->bs; a.l_valid = d->l_valid;
   a.mask = d->mask;
-  // (few entries in all, since each group also counts those before it)
-  if (lay.n <= kIdxSmallEntries && d->nblk <= kIdxSmallBlocks) {
-    const size_t lds = (2 * 1024 + 16) * 4 + (size_t)(d->nblk * d->kk) * 2;
-    hipLaunchKernelGGL(small_index_kernel, dim3((unsigned)(d->B * d->hsel)), dim3(1024), lds, s, a,
+  if (small_index_fits(d, lay.n)) {
+    const size_t lds = (size_t)kIdxWaves * (d->nblk + 2) * 4 + (size_t)lay.n * 2;
+    const int e = lds_optin((const void *)small_index_kernel, lds, "hipFuncSetAttribute(small_index)");
+    if (e) return e;
+    hipLaunchKernelGGL(small_index_kernel, dim3((unsigned)(d->B * d->hsel)), dim3(kIdxWaves * 64), lds, s, a,
                        (int32_t *)(ws + lay.vals_out), (int32_t *)(ws + lay.seg_off));
     return hip_check(hipGetLastError(), "small_index_kernel launch");
   }
