@@ -84,14 +84,14 @@ def block_mass(q, k, bs, scale=None):
 
 def _block_list(selector, q, k):
     """selector.select(q, k); for the Quest selectors below without the round
-    trip through int64 (only when the instance's select is the class's own)."""
-    fn = getattr(selector.select, "__func__", None)
-    if fn is not None and selector.select.__self__ is selector:
-        for cls in (SelectMax, SelectLastTok, SelectMaxQMax, SelectTwoStage):
-            if type(selector) is cls and fn is cls.select:
-                with torch.no_grad():
-                    return selector._select32(q, k)
-    return selector.select(q, k)
+    trip through int64, as long as the instance's select is the one defined here
+    (one set on the instance, its class or a subclass is called)."""
+    own = _QUEST_SELECT.get(type(selector))
+    fn = selector.select
+    if own is not None and getattr(fn, "__func__", None) is own and fn.__self__ is selector:
+        with torch.no_grad():
+            return selector._select32(q, k)
+    return fn(q, k)
 
 
 def _finish(score, topk, sink, B, Hkv, nblk, dev):
@@ -176,6 +176,10 @@ class SelectTwoStage:
 
     def _select32(self, q, k):
         return selection.select_two_stage(q, k, self.bs, self.topk, sink=self.sink, over=self.over)
+
+
+# their select functions as defined above: one that replaces them later is not equal to these
+_QUEST_SELECT = {cls: cls.select for cls in (SelectMax, SelectLastTok, SelectMaxQMax, SelectTwoStage)}
 
 
 class SelectLearned:
