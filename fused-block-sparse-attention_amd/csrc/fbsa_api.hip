@@ -50,6 +50,18 @@ static int64_t esize(int dtype) { return dtype == FBSA_F32 ? 4 : 2; }
 
 static bool aligned(const void *p, int64_t a) { return ((uintptr_t)p % (uintptr_t)a) == 0; }
 
+// The attention kernels copy tiles of consecutive rows with 32-bit byte offsets
+// from the tile's first row (at most 64 rows), so those rows' span must fit.
+static int check_row_span(const fbsa_attn_desc *d, int64_t stride, int64_t limit, const char *name, const char *fn) {
+  const int64_t es = esize(d->dtype), most = d->dtype == FBSA_F32 && d->D >= 128 ? 16 : (d->D >= 256 ? 32 : 64);
+  const int64_t rows = d->bs < most ? d->bs : most;
+  if ((rows - 1) * stride * es + d->D * es > limit)
+    return fail(FBSA_EUNSUPPORTED, "%s: %s row stride of %lld elements: %lld rows span more than %lld bytes", fn, name,
+                (long long)stride, (long long)rows, (long long)limit);
+  return FBSA_OK;
+}
+static constexpr int64_t kSpan = 0x100000000LL;
+
 // Shape and layout checks shared by the attention entry points.
 static int check_attn(const fbsa_attn_desc *d, const char *fn) {
   if (!d) return fail(FBSA_EINVAL, "%s: null descriptor", fn);
@@ -89,7 +101,9 @@ static int check_attn(const fbsa_attn_desc *d, const char *fn) {
   for (int t = 0; t < 5; ++t)
     if (rs[t] * es >= 0x100000000LL)
       return fail(FBSA_EUNSUPPORTED, "%s: a row stride of %lld elements is 4 GiB or more", fn, (long long)rs[t]);
-  return FBSA_OK;
+  int e = check_row_span(d, d->sk[2], kSpan, "k", fn);
+  if (!e) e = check_row_span(d, d->sv[2], kSpan, "v", fn);
+  return e;
 }
 
 // FBSA_FLAG_DENSE: the implicit all-blocks list (kk = nblk, no sel, no gate).
@@ -175,6 +189,7 @@ int fbsa_block_mass(const fbsa_attn_desc *d, const void *q, const void *k, float
   if (!q || !k || !mass || !ws) return fail(FBSA_EINVAL, "fbsa_block_mass: null pointer");
   if (!aligned(q, 16) || !aligned(k, 16) || !aligned(mass, 4) || !aligned(ws, 16))
     return fail(FBSA_EINVAL, "fbsa_block_mass: misaligned pointer");
+  if ((e = check_row_span(d, d->sk[2], kSpan / 2, "k", "fbsa_block_mass"))) return e;  // its offsets are signed
   return run_block_mass(d, q, k, mass, ws, (hipStream_t)stream);
 }
 
@@ -335,6 +350,9 @@ static int check_bwd(const fbsa_attn_desc *d, const char *fn, BwdLayout *lay, co
   if (e) return e;
   if (d->flags & ~(FBSA_FLAG_OUT_GATE | FBSA_FLAG_DENSE | FBSA_FLAG_DGATE | FBSA_FLAG_RAGGED)) return fail(FBSA_EINVAL, "%s: unknown flags 0x%x", fn, d->flags);
   if ((d->flags & FBSA_FLAG_DENSE) && (e = check_dense(d, nullptr, nullptr, fn))) return e;
+  if ((e = check_row_span(d, d->sq[2], kSpan, "q", fn))) return e;
+  // (with an output gate the kernels copy the workspace's rows instead of dout's)
+  if (!(d->flags & FBSA_FLAG_OUT_GATE) && (e = check_row_span(d, d->sdo[2], kSpan, "dout", fn))) return e;
   e = bwd_layout(d, lay);
   if (e) return e;
   if (!ws || !aligned(ws, 256)) return fail(FBSA_EINVAL, "%s: workspace must be non-null and 256-byte aligned", fn);

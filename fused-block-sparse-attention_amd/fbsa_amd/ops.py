@@ -50,9 +50,10 @@ def _require_cuda(*ts):
 
 def _kernel_ready(x, min_align=16):
     """Unit stride on D, row starts and base 16-byte aligned (the kernels load
-    rows with 16-byte vector / direct-to-LDS loads); copy otherwise."""
+    rows with 16-byte vector / direct-to-LDS loads), rows less than 32 MiB apart
+    (a copy's offset within a chunk of up to 64 rows has 32 bits); copy otherwise."""
     es = x.element_size()
-    ok = x.stride(-1) == 1 and x.data_ptr() % min_align == 0 and all(
+    ok = x.stride(-1) == 1 and x.data_ptr() % min_align == 0 and x.stride(-2) * es < 1 << 25 and all(
         (s * es) % 16 == 0 for s in x.stride()[:-1])
     return x if ok else x.contiguous()
 
