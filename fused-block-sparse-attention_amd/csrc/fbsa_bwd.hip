@@ -35,8 +35,17 @@
 // dS = P (dP - D), dQ = dS K scale, dK = dS^T Q scale, dV = P^T dO), the
 // token-causal/padding/duplicate masks of src/qwen_blocksparse.py:67-72, and
 // the gate gradient the gather path (src/ssa_model.py:72-74) gives.
+// dQ and dK/dV of tensors that end inside the last block (FBSA_FLAG_RAGGED) are
+// instantiations of their own, compiled by fbsa_bwd_ragged.hip from this file;
+// it leaves out everything else.
+#ifndef FBSA_BWD_RAGGED
+#define FBSA_BWD_RAGGED 0
+#endif
+
+#if !FBSA_BWD_RAGGED
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
+#endif
 
 #include "fbsa_common.h"
 #include "fbsa_internal.h"
@@ -108,6 +117,8 @@ enum { KIND_FULL = 0, KIND_DIAG = 1, KIND_ABS = 2, KIND_PAD = 3 };
 #define FBSA_DKDV_LDS_BUDGET 40960
 #endif
 
+
+#if !FBSA_BWD_RAGGED
 static int64_t esize(int dtype) { return dtype == FBSA_F32 ? 4 : 2; }
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -225,6 +236,8 @@ int bwd_layout(const fbsa_attn_desc *d, BwdLayout *lay) {
   return FBSA_OK;
 }
 
+#endif  // !FBSA_BWD_RAGGED
+
 // ----------------------------------------------------------------- stage 1
 // Row statistics (workspace and LDS): rows 4k .. 4k + 3 keep their four
 // -lse * log2 e at floats 8k .. 8k + 3 and their four -delta at 8k + 4 .. 8k + 7
@@ -237,17 +250,6 @@ __device__ __forceinline__ int64_t rs_delta_at(int64_t row) { return (row >> 2) 
 __device__ __forceinline__ float rs_lse(const float *M, int k4, int r) { return M[k4 * 8 + r]; }
 __device__ __forceinline__ float rs_delta(const float *M, int k4, int r) { return M[k4 * 8 + 4 + r]; }
 
-struct PrepArgs {
-  const void *o, *dout, *og;
-  const float *lse;
-  float *rowstat;
-  void *dout_attn, *dout_gate;
-  int64_t Hq, L, rows;
-  int64_t so[3], sdo[3], sog[3];
-  int64_t held;  // rows per head that o, dout and out_gate hold (below L: ragged)
-  int og_vec;  // out-gate rows and dout_gate 16-byte aligned: vector loads and stores
-};
-
 template <typename T> __device__ __forceinline__ float half_to_f32(uint32_t h) {
   if constexpr (__is_same(T, bf16)) {
     return __uint_as_float(h << 16);
@@ -258,6 +260,18 @@ template <typename T> __device__ __forceinline__ float half_to_f32(uint32_t h) {
     return (float)x;
   }
 }
+
+#if !FBSA_BWD_RAGGED
+struct PrepArgs {
+  const void *o, *dout, *og;
+  const float *lse;
+  float *rowstat;
+  void *dout_attn, *dout_gate;
+  int64_t Hq, L, rows;
+  int64_t so[3], sdo[3], sog[3];
+  int64_t held;  // rows per head that o, dout and out_gate hold (below L: ragged)
+  int og_vec;  // out-gate rows and dout_gate 16-byte aligned: vector loads and stores
+};
 
 template <typename T> __device__ __forceinline__ void load8f(const T *p, float *v) {
   if constexpr (sizeof(T) == 4) {
@@ -616,6 +630,8 @@ int run_transpose_index(const fbsa_attn_desc *d, const BwdLayout &lay, const int
   return hip_check(hipGetLastError(), "seg_off_kernel launch");
 }
 
+#endif  // !FBSA_BWD_RAGGED
+
 // ----------------------------------------------------------------- stages 3, 4
 struct BwdArgs {
   const void *q, *k, *v, *dout;  // dout: gradient of the un-gated attention output
@@ -643,6 +659,9 @@ struct BwdArgs {
   int mask, grp;
   int dense;  // FBSA_FLAG_DENSE: slot s is block s; lists implicit (i = j + position when causal)
 };
+
+// the RAGGED instantiations (fbsa_bwd_ragged.hip)
+int bwd_dispatch_ragged(const fbsa_attn_desc *d, const BwdArgs &a, bool dq, hipStream_t s);
 
 // ROWS: the block rows one workgroup owns (one wave per 16), BS unless a
 // block is split over several workgroups.
@@ -677,7 +696,10 @@ template <typename T, int BS, int D> constexpr int dq_minwg() {
 
 // DG: the gate gradient is asked for (its sums and the slot masses are
 // compiled into the chunk loop only then)
-template <typename T, int BS, int D, bool DENSE = false, bool DG = false>
+// RAGGED: the tensors end inside the last block; copies past the end are limited
+// to its last row, which whole-length launches do without (training steps of 32 x
+// 1024 tokens 289 -> 283 us, of 262144 tokens 4012 -> 3987 us)
+template <typename T, int BS, int D, bool DENSE, bool DG, bool RAGGED>
 __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdArgs a) {
   using C = BwdCfg<T, BS, D, FBSA_DQ_LDS_BUDGET, 0>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -780,7 +802,7 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
   const int64_t qpos = i * BS + tq;
   // (a row past the tensors' end takes the last one's values; its lse of -inf
   // makes its P zero, and nothing of it is stored)
-  const int64_t qr = qpos < a.rows ? qpos : a.rows - 1;
+  const int64_t qr = !RAGGED || qpos < a.rows ? qpos : a.rows - 1;
   RowFrag<T, D> qf, df;
   qf.load((const T *)a.q + b * a.sq[0] + hq * a.sq[1] + qr * a.sq[2], g);
   df.load((const T *)a.dout + b * a.sdo[0] + hq * a.sdo[1] + qr * a.sdo[2], g);
@@ -829,11 +851,13 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
     f_gate = DENSE ? 0.f : s_gate[sc];
   };
   auto issue = [&]() {
-    const uint32_t row0 = tail_row((uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC), (uint32_t)a.rows);
-    plan.issue((unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES, (const char *)(kbase + (int64_t)row0 * a.sk[2]),
-               (const char *)(vbase + (int64_t)row0 * a.sv[2]),
-               tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)(a.sk[2] * C::ES), D * C::ES),
-               tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)(a.sv[2] * C::ES), D * C::ES), w);
+    const uint32_t first = (uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC);
+    const uint32_t row0 = RAGGED ? tail_row(first, (uint32_t)a.rows) : first;
+    plan.template issue<RAGGED>(
+        (unsigned)(uintptr_t)stages + ist * C::STAGE_BYTES, (const char *)(kbase + (int64_t)row0 * a.sk[2]),
+        (const char *)(vbase + (int64_t)row0 * a.sv[2]),
+        RAGGED ? tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)(a.sk[2] * C::ES), D * C::ES) : 0,
+        RAGGED ? tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)(a.sv[2] * C::ES), D * C::ES) : 0, w);
     ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
     if (++ich == C::NCH) { ich = 0; ++islot; }
   };
@@ -1003,7 +1027,7 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
   T *dqrow = (T *)a.dq + ((b * a.Hq + hq) * a.rows + qpos) * D;
 #pragma unroll
   for (int mt = 0; mt < D / 16; ++mt) {
-    if (qpos >= a.rows) break;
+    if (RAGGED && qpos >= a.rows) break;
     const int d0 = 16 * mt + 4 * g;
     if constexpr (sizeof(T) == 4) {
       *(f32x4 *)(dqrow + d0) = f32x4{dqacc[mt][0] * a.scale, dqacc[mt][1] * a.scale, dqacc[mt][2] * a.scale,
@@ -1106,7 +1130,7 @@ template <typename T, int BS, int D> constexpr bool dkdv_unrolled() {
 // exponentials), so occupancy decides: for bs 64 with 16-bit d <= 64 the
 // kernel is held to four waves per SIMD (at most 128 VGPRs) and its two-stage
 // ring (35 KB of LDS) fits four workgroups per CU.
-template <typename T, int BS, int D, bool DENSE = false>
+template <typename T, int BS, int D, bool DENSE, bool RAGGED>
 __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>())) void dkdv_kernel(BwdArgs a) {
   using C = DkdvCfg<T, BS, D>;
   constexpr bool SPLIT = FBSA_BWD_SPLIT && sizeof(T) == 2;
@@ -1183,7 +1207,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
   const int role = ROLES == 2 ? (w & 1) : 0, kw = ROLES == 2 ? (w >> 1) : w;
   const int u = kpart * KEYS + kw * 16 + p;  // this lane's key row within block j (B-operand column)
   const int64_t kpos = j * BS + u;
-  const int64_t kr = kpos < a.rows ? kpos : a.rows - 1;  // (a key past the tensors' end is masked and not stored)
+  const int64_t kr = !RAGGED || kpos < a.rows ? kpos : a.rows - 1;  // (a key past the tensors' end is masked and not stored)
   const T *krow = (const T *)a.k + b * a.sk[0] + hk * a.sk[1] + kr * a.sk[2];
   const T *vrow = (const T *)a.v + b * a.sv[0] + hk * a.sv[1] + kr * a.sv[2];
   RowFrag<T, D> kf, vf;  // two roles: kf holds K (role 0) or V (role 1), vf is unused
@@ -1281,7 +1305,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
         // addresses below are formed by scalar instructions
         const uint32_t row0 =
             (uint32_t)__builtin_amdgcn_readfirstlane(f_iq) * (uint32_t)BS + (uint32_t)(ic * C::KC);
-        const uint32_t trow = tail_row(row0, (uint32_t)a.rows);
+        const uint32_t trow = RAGGED ? tail_row(row0, (uint32_t)a.rows) : row0;
         const char *qb = qh + (uint64_t)trow * qrs;
         const char *db = dh + (uint64_t)trow * drs;
         const unsigned st = (unsigned)(uintptr_t)stages + istg * C::STAGE_BYTES;
@@ -1289,8 +1313,8 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
         const uint32_t dl = tail_limit<C::KC>(trow, (uint32_t)a.rows, drs, D * C::ES);
   #pragma unroll
         for (int n = 0; n < C::LPT; ++n) {
-          const uint32_t lim = tdo[n] ? dl : ql;
-          g2lds16_s(tdo[n] ? db : qb, (uint32_t)toff[n] < lim ? (uint32_t)toff[n] : lim, st + (n * C::NW + w) * 1024);
+          const uint32_t lim = tdo[n] ? dl : ql, off = (uint32_t)toff[n];
+          g2lds16_s(tdo[n] ? db : qb, RAGGED && off > lim ? lim : off, st + (n * C::NW + w) * 1024);
         }
         // wave w copies rows w KC/NW .. (w + 1) KC/NW - 1 of the row statistics (two per lane)
         if (lane < C::KC / (2 * C::NW))
@@ -1628,7 +1652,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
     }
     return;
   }
-  if (kpos >= a.rows) return;
+  if (RAGGED && kpos >= a.rows) return;
   if constexpr (ROLES == 2) {
     T *row = (T *)(role ? a.dk : a.dv) + ((b * a.Hkv + hk) * a.rows + kpos) * D;
     const float sc = role ? a.scale : 1.f;
@@ -1663,6 +1687,7 @@ __global__ __launch_bounds__((dkdv_rows<T, BS, D>() * 4), (dkdv_minwg<T, BS, D>(
   }
 }
 
+#if !FBSA_BWD_RAGGED
 // List segments. Work item wi = (b, KV head, key block) walks the transposed
 // list of its selection head; longer than E entries it is cut into
 // S = ceil(len / E) segments. cnt[wi] = (S - 1) << 32 | S for a split item, 0
@@ -1807,6 +1832,8 @@ static void fill_bwd(const fbsa_attn_desc *d, const BwdLayout &lay, char *ws, Bw
   if (a.dense) a.ent = nullptr;
 }
 
+#endif  // !FBSA_BWD_RAGGED
+
 template <typename K> static int set_lds(K kern, size_t lds, const char *what) {
   if (lds > 160 * 1024 - 64) return fail(FBSA_EUNSUPPORTED, "%s needs %zu bytes of LDS", what, lds);
   return lds_optin((const void *)kern, lds, "hipFuncSetAttribute(bwd)");
@@ -1819,9 +1846,9 @@ template <typename T, int BS, int D, bool DENSE, bool DG> static int launch_dq_a
   // per-row scratch
   const size_t lds = (size_t)C::NSTAGE * C::STAGE_BYTES +
                      (DENSE ? 0 : (size_t)a.kk * (DG ? 16 : 12) + (DG ? (2 * C::NW + BS) * 4 : 0));
-  int e = set_lds(dq_kernel<T, BS, D, DENSE, DG>, lds, "fbsa_bwd_dq");
+  int e = set_lds(dq_kernel<T, BS, D, DENSE, DG, FBSA_BWD_RAGGED != 0>, lds, "fbsa_bwd_dq");
   if (e) return e;
-  hipLaunchKernelGGL((dq_kernel<T, BS, D, DENSE, DG>), dim3((unsigned)(a.B * a.Hq * a.nblk)), dim3(C::NT), lds, s, a);
+  hipLaunchKernelGGL((dq_kernel<T, BS, D, DENSE, DG, FBSA_BWD_RAGGED != 0>), dim3((unsigned)(a.B * a.Hq * a.nblk)), dim3(C::NT), lds, s, a);
   return hip_check(hipGetLastError(), "dq_kernel launch");
 }
 
@@ -1832,10 +1859,10 @@ template <typename T, int BS, int D, bool DENSE> static int launch_dkdv_as(const
                          ? (size_t)(dkdv_pipe<T, BS, D>() ? 2 : 1) * (dkdv_keys<T, BS, D>() / 16) * 64 * (HR / 16) * 16
                          : 0;
   const size_t lds = (size_t)C::NSTAGE * C::STAGE_BYTES + 128 * 16 + xch;
-  int e = set_lds(dkdv_kernel<T, BS, D, DENSE>, lds, "fbsa_bwd_dkdv");
+  int e = set_lds(dkdv_kernel<T, BS, D, DENSE, FBSA_BWD_RAGGED != 0>, lds, "fbsa_bwd_dkdv");
   if (e) return e;
   const int64_t nwg = (a.B * a.Hkv * a.nblk + (a.wi_slot ? a.seg_entries_xub : 0)) * (BS / dkdv_keys<T, BS, D>());
-  hipLaunchKernelGGL((dkdv_kernel<T, BS, D, DENSE>), dim3((unsigned)nwg), dim3(C::NT), lds, s, a);
+  hipLaunchKernelGGL((dkdv_kernel<T, BS, D, DENSE, FBSA_BWD_RAGGED != 0>), dim3((unsigned)nwg), dim3(C::NT), lds, s, a);
   return hip_check(hipGetLastError(), "dkdv_kernel launch");
 }
 
@@ -1869,7 +1896,12 @@ template <typename T> static int bwd_bs(const BwdArgs &a, int64_t bs, int64_t D,
   return fail(FBSA_EUNSUPPORTED, "fbsa_bwd: block size %lld not in {16,32,64,128}", (long long)bs);
 }
 
+#if FBSA_BWD_RAGGED
+int bwd_dispatch_ragged(const fbsa_attn_desc *d, const BwdArgs &a, bool dq, hipStream_t s) {
+#else
 static int bwd_dispatch(const fbsa_attn_desc *d, const BwdArgs &a, bool dq, hipStream_t s) {
+  if (a.rows < a.L) return bwd_dispatch_ragged(d, a, dq, s);
+#endif
   switch (d->dtype) {
     case FBSA_BF16: return bwd_bs<bf16>(a, d->bs, d->D, dq, s);
     case FBSA_F16: return bwd_bs<f16>(a, d->bs, d->D, dq, s);
@@ -1878,6 +1910,7 @@ static int bwd_dispatch(const fbsa_attn_desc *d, const BwdArgs &a, bool dq, hipS
   return fail(FBSA_EINVAL, "fbsa_bwd: bad dtype %d", d->dtype);
 }
 
+#if !FBSA_BWD_RAGGED
 int run_bwd_dq(const fbsa_attn_desc *d, const BwdLayout &lay, const void *q, const void *k, const void *v,
                const void *dout, const int32_t *sel, const float *gate, void *dq, float *dgate, char *ws,
                hipStream_t s, const void *o, const float *lse) {
@@ -1955,5 +1988,7 @@ int run_bwd_dkdv(const fbsa_attn_desc *d, const BwdLayout &lay, const void *q, c
   }
   return hip_check(hipGetLastError(), "dkdv_reduce_kernel launch");
 }
+
+#endif  // !FBSA_BWD_RAGGED
 
 }  // namespace fbsa

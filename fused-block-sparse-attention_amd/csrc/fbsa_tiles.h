@@ -316,13 +316,14 @@ template <typename T, int KC, int D, int NW, int LPT> struct TilePairPlan {
     }
   }
   // st: the stage's LDS address; src0 / src1: the first rows of the chunk (wave-uniform);
-  // lim0 / lim1: tail_limit of either
+  // lim0 / lim1: tail_limit of either (LIM only)
+  template <bool LIM>
   __device__ __forceinline__ void issue(unsigned st, const char *src0, const char *src1, uint32_t lim0, uint32_t lim1, int w) const {
 #pragma unroll
     for (int n = 0; n < LPT; ++n) {
       const char *base = part[n] ? src1 : src0;
       const uint32_t lim = part[n] ? lim1 : lim0;
-      g2lds16_s(base, off[n] < lim ? off[n] : lim, st + (n * NW + w) * 1024);
+      g2lds16_s(base, LIM && off[n] > lim ? lim : off[n], st + (n * NW + w) * 1024);
     }
   }
 };

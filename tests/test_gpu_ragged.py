@@ -24,7 +24,9 @@ def _run(q, k, v, sel, og, do, gate, mask, L, bs, ragged):
 @pytest.mark.parametrize("extra", ["plain", "out_gate", "gate", "dense", "none"])
 @pytest.mark.parametrize("dtype,D,bs,nblk,last", [("bf16", 256, 128, 5, 1), ("bf16", 64, 64, 6, 63), ("f16", 128, 128, 3, 65),
                                                   ("f16", 256, 64, 4, 33), ("bf16", 32, 16, 7, 5), ("f32", 64, 64, 5, 17),
-                                                  ("f32", 256, 128, 3, 15), ("bf16", 64, 32, 1, 7)])
+                                                  ("f32", 256, 128, 3, 15), ("bf16", 64, 32, 1, 7),
+                                                  ("bf16", 128, 64, 5, 7), ("f16", 64, 128, 4, 127), ("f32", 128, 128, 3, 1),
+                                                  ("f32", 32, 16, 9, 3)])
 def test_ragged_equals_padded(dtype, D, bs, nblk, last, extra):
     from fbsa_amd import ops
     dt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
