@@ -246,11 +246,10 @@ __global__ __launch_bounds__(256) void pool_kernel(PoolArgs a) {
 // are issued back to back (fixed trip count; rows past l_valid are read at a
 // clamped address and contribute 0). MEAN_TOK_THEN_GRP gives each wave whole
 // heads; the other ops split the block's tokens over the waves and, where the
-// blocks alone are few (below), a row wider than 64 elements over workgroups
-// (DC = 8 chunks each, 128 bytes of a 16-bit row; a.D / 64 slices of a block
-// back to back).
+// blocks alone are few (launch_pool_op), a row over workgroups (SLICED: DC chunks
+// each, the slices of a block back to back).
 // Workgroups [0, nwg0) pool a0, the rest pool a1 (two tensors in one launch).
-template <typename T, int DC, int BS, int OP>
+template <typename T, int DC, int BS, int OP, bool SLICED = false>
 __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1, int64_t nwg0) {
   constexpr int NW = 4, TLW = 64 / DC;
   constexpr int RPH = BS >= TLW ? BS / TLW : 1;            // rows per lane per head (whole block in one wave)
@@ -263,7 +262,7 @@ __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1
   // 32-bit index arithmetic (launch indices are below 2^31)
   uint32_t blk = second ? blockIdx.x - (uint32_t)nwg0 : blockIdx.x;
   int d0 = 0;  // first element of this workgroup's slice of the row
-  if constexpr (op != FBSA_POOL_MEAN_TOK_THEN_GRP) {
+  if constexpr (SLICED) {
     const uint32_t ns = (uint32_t)a.D / (8 * DC);
     d0 = (int)(blk % ns) * (8 * DC);
     blk /= ns;
@@ -314,9 +313,28 @@ __global__ __launch_bounds__(256) void pool_wave_kernel(PoolArgs a0, PoolArgs a1
 #pragma unroll
       for (int e = 0; e < 8; ++e) r0[e] += (double)round_dt<T>(acc[e] / (double)BS);
     }
+  } else if constexpr (op == FBSA_POOL_MEAN_GRP_THEN_TOK && !SLICED) {
+    // tokens split over waves and lanes; per token an exact group sum, rounded mean
+    for (int n = 0; n < RPW; ++n) {
+      const int t = (w + n * NW) * TLW + tl;
+      double g[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) g[e] = 0.0;
+#pragma unroll 8
+      for (int64_t hh = 0; hh < a.grp; ++hh) {
+        double v[8];
+        load8<T>(rowptr(ho * a.grp + hh, t), v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) g[e] += v[e];
+      }
+      const bool ok = t < nval && t < BS;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r0[e] += ok ? (double)round_dt<T>(mean_div(g[e], a.grp)) : 0.0;
+    }
+    xor_sum(r0);
   } else if constexpr (op == FBSA_POOL_MEAN_GRP_THEN_TOK) {
-    // tokens split over waves and lanes; per token an exact group sum, rounded
-    // mean. A lane's (token, head) rows in order, eight loads in flight.
+    // the same sums for few workgroups: a lane's (token, head) rows in order,
+    // eight loads in flight (on a full GPU the bookkeeping costs 8 to 25%)
     double g[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) g[e] = 0.0;
@@ -553,8 +571,10 @@ __global__ __launch_bounds__(256) void pool_grp_kernel(PoolArgs a, int64_t n) {
   }
 }
 
-// SC: 16-byte chunks of a workgroup's slice of the row (token-split ops)
+// SC: chunks of a workgroup's slice of the row (token-split ops; DC: whole rows)
 template <typename T, int DC, int BS, int SC> static void launch_pool_sliced(const PoolArgs &a, int64_t nwg, hipStream_t s) {
+  constexpr bool SL = SC != DC;
+  const int64_t n = nwg * (DC / SC);
   switch (a.op) {
     case FBSA_POOL_MEAN_TOK_THEN_GRP:
       if (a.grp == 1) {
@@ -565,26 +585,34 @@ template <typename T, int DC, int BS, int SC> static void launch_pool_sliced(con
                          a, nwg);
       return;
     case FBSA_POOL_MEAN_GRP_THEN_TOK:
-      hipLaunchKernelGGL((pool_wave_kernel<T, SC, BS, FBSA_POOL_MEAN_GRP_THEN_TOK>), dim3((unsigned)(nwg * (DC / SC))),
-                         dim3(256), 0, s, a, a, nwg * (DC / SC));
+      hipLaunchKernelGGL((pool_wave_kernel<T, SC, BS, FBSA_POOL_MEAN_GRP_THEN_TOK, SL>), dim3((unsigned)n), dim3(256), 0, s,
+                         a, a, n);
       return;
     default:  // MAX / MIN / MINMAX share one instantiation (the op picks the outputs)
-      hipLaunchKernelGGL((pool_wave_kernel<T, SC, BS, FBSA_POOL_MINMAX>), dim3((unsigned)(nwg * (DC / SC))), dim3(256), 0,
-                         s, a, a, nwg * (DC / SC));
+      hipLaunchKernelGGL((pool_wave_kernel<T, SC, BS, FBSA_POOL_MINMAX, SL>), dim3((unsigned)n), dim3(256), 0, s, a, a, n);
       return;
   }
 }
 
+// A workgroup walks its BS x grp rows in serial steps, so few workgroups leave
+// the memory idle and a row is then split over several; with enough of them
+// whole rows read better. A slice is no narrower than lets one step of the
+// workgroup (256 / SC rows) fit the block. Measured (us, whole rows -> slices;
+// blocks of 128, d 256, bf16): group mean of 16 heads over 2, 64 blocks 32 -> 14,
+// 256 48 -> 25, 512 60 -> 47, but 1024 102 -> 111; of 2 heads over 1, 64 blocks 18
+// -> 6, 256 19 -> 11; at d 128 256 blocks 11 -> 8, 512 (fp32) 22 -> 23. Min / max
+// has a head's rows only: 32 blocks 5.2 -> 4.4, 64 5.3 -> 6.0, and with shorter
+// blocks slices are always behind (64 tokens, 255 blocks 4.6 -> 15).
 template <typename T, int DC, int BS> static void launch_pool_op(const PoolArgs &a, int64_t nwg, hipStream_t s) {
-  // Slices of 8 chunks while whole-row workgroups are fewer than four per CU, of
-  // 4 (64 bytes of a 16-bit row) while they are fewer than one: a workgroup walks its BS x grp rows in serial steps of eight loads, so few of
-  // them leave the memory idle (group mean of 16 heads over 2, d 256, blocks of
-  // 128: 1999 tokens, 32 blocks, 50 -> 11 us, 18 in slices of 8; 16301 tokens,
-  // 256 blocks, 82 -> 39 us). With more, whole rows read better (65536 tokens, 1024 blocks: min /
-  // max 16 us whole, 22 us in slices).
-  if (DC > 4 && nwg < 256) launch_pool_sliced<T, DC, BS, (DC > 4 ? 4 : DC)>(a, nwg, s);
-  else if (DC > 8 && nwg < 1024) launch_pool_sliced<T, DC, BS, (DC > 8 ? 8 : DC)>(a, nwg, s);
-  else launch_pool_sliced<T, DC, BS, DC>(a, nwg, s);
+  constexpr int S = BS >= 64 ? 4 : (BS >= 32 ? 8 : 16), W = S < 8 ? 8 : S;
+  if (a.op == FBSA_POOL_MEAN_GRP_THEN_TOK) {
+    if (DC > S && nwg <= 128) return launch_pool_sliced<T, DC, BS, (DC > S ? S : DC)>(a, nwg, s);
+    const int64_t most = DC == 32 && BS >= 64 && sizeof(T) == 2 ? 512 : (DC == 32 || BS >= 64 ? 256 : 0);
+    if (DC > W && nwg <= most) return launch_pool_sliced<T, DC, BS, (DC > W ? W : DC)>(a, nwg, s);
+  } else if (a.op != FBSA_POOL_MEAN_TOK_THEN_GRP && BS >= 128 && DC > 4 && nwg * (DC / 4) <= 256) {
+    return launch_pool_sliced<T, DC, BS, (DC > 4 && BS >= 128 ? 4 : DC)>(a, nwg, s);
+  }
+  launch_pool_sliced<T, DC, BS, DC>(a, nwg, s);
 }
 
 template <typename T, int DC> static bool launch_pool_bs(const PoolArgs &a, int64_t nwg, hipStream_t s) {

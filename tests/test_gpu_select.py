@@ -78,6 +78,62 @@ def test_pool_quest_exact(dtype):
     assert np.array_equal(np64(kmin), rmin) and np.array_equal(np64(kmax), rmax)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("bs,D,nblk", [(16, 64, 100), (16, 128, 100), (16, 256, 128), (16, 256, 129), (16, 256, 257),
+                                       (32, 64, 100), (32, 128, 128), (32, 128, 129), (32, 256, 256), (32, 256, 257),
+                                       (64, 64, 128), (64, 64, 129), (64, 128, 128), (64, 128, 129), (64, 128, 257),
+                                       (64, 256, 128), (64, 256, 129), (64, 256, 512), (64, 256, 513),
+                                       (128, 64, 128), (128, 64, 129), (128, 128, 64), (128, 128, 65), (128, 256, 32),
+                                       (128, 256, 33)])
+def test_pool_slices_exact(dtype, bs, D, nblk):
+    # group-mean and min / max pooling split a row over workgroups while blocks are few: both
+    # sides of every line of launch_pool_op, with a short last block
+    from fbsa_amd import selection
+    g = torch.Generator().manual_seed(nblk + D)
+    x = randn(g, (1, 3, nblk * bs - 5, D), dtype)
+    _say("pool slices", dtype, bs, D, nblk)
+    got = selection.pool(x.to(DEV), bs, "mean_grp_then_tok", grp=3)
+    assert np.array_equal(np64(got), osel.pool_mean_grp_then_tok(np64(x), 1, bs, dtype))
+    kmin, kmax = selection.pool(x[:, :1].to(DEV), bs, "minmax")
+    rmin, rmax = osel.pool_minmax(np64(x[:, :1]), bs)
+    assert np.array_equal(np64(kmin), rmin) and np.array_equal(np64(kmax), rmax)
+
+
+def _us(run, n=20):
+    """Median of five timings of n calls back to back, in us a call."""
+    run()
+    t = []
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(n):
+            run()
+        b.record()
+        b.synchronize()
+        t.append(a.elapsed_time(b) * 1000 / n)
+    return sorted(t)[2]
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("op,grp,D,bs,nblk", [("minmax", 1, 256, 32, 1000), ("minmax", 1, 256, 64, 255), ("minmax", 1, 128, 64, 512),
+                                              ("mean_grp_then_tok", 2, 256, 16, 1000), ("mean_grp_then_tok", 3, 128, 16, 512),
+                                              ("mean_grp_then_tok", 2, 256, 16, 255)])
+def test_pool_time_near_the_token_mean(dtype, op, grp, D, bs, nblk):
+    # the same bytes as a token mean, whose workgroups always read whole rows: at most twice its
+    # time (and a launch) where slices of the rows would be three times behind
+    from fbsa_amd import _lib, selection
+    x = torch.zeros(1, grp, nblk * bs, D, device=DEV, dtype={"bf16": torch.bfloat16, "f32": torch.float32}[dtype])
+    out, out2 = (torch.empty(1, 1, nblk, D, device=DEV, dtype=x.dtype) for _ in range(2))
+    lib, s = _lib.load(), torch.cuda.current_stream().cuda_stream
+
+    def call(o):
+        d = selection._pool_desc(x, bs, o, grp, None)
+        return lambda: _lib.check(lib.fbsa_pool(d, x.data_ptr(), out.data_ptr(), out2.data_ptr(), s), "pool")
+    _say("pool time", dtype, op, grp, D, bs, nblk)
+    t, ref = _us(call(op)), _us(call("mean_tok_then_grp"))
+    assert t <= 2 * ref + 2, (t, ref)
+
+
 def _check_sel(got, ref, what):
     got = np.asarray(got)
     ref = np.asarray(ref)
