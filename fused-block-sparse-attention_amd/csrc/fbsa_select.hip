@@ -1927,17 +1927,35 @@ static void sel_chunking(int64_t B, int64_t H, int64_t nblk, bool tri, int64_t o
   *nch = (ntiles + c - 1) / c;
 }
 
-// Up to kSelRowMax candidate blocks a wave per row (select_row_kernel) finishes
-// first. Measured (select alone, us, MFMA engine -> row kernel, bf16 d 64): 1 x
-// 64 blocks 29 -> 5, 32 x 32 31 -> 4, 1 x 256 39 -> 11, 16 x 256 39 -> 19; past
-// kSelRowPairs (row, candidate) pairs the MFMA engine is ahead again (64 x 256:
-// 40 -> 51). Against select_kernel (fp32, d 64): 1 x 64 41 -> 6, 1 x 256 55 ->
-// 13, 64 x 256 150 -> 95.
+// Up to kSelRowMax candidate blocks a wave per row (select_row_kernel) is often
+// the quickest engine, and loses where its waves, which each read their own
+// candidates, read too much: many rows of wide operands. The choice compares
+// estimates of the engines' times in us, fitted to measurements over 8 to 256
+// blocks, 64 to 260000 rows, d 16 to 256, both widths, all scores and budgets 8
+// to 62 (row and select_kernel to 15 and 20% rms over 426 shapes; of these 8 end
+// up more than 10% behind the better engine of the two, at most 31%).
+// Measured, other engine -> row kernel: MFMA (bf16, budget 8) 1 x 64 blocks 29 -> 5,
+// 8 x 256 d 32 31 -> 9, 128 x 128 d 32 29 -> 25, 128 x 128 d 64 MAX2 39 -> 64;
+// select_kernel (fp32) d 16 512 x 64 MAX2 158 -> 37, d 64 64 x 256 125 -> 95, d 256
+// (budget 8) 8 x 256 QUEST 77 -> 117, 32 x 256 MAX2 154 -> 424.
 constexpr int64_t kSelRowMax = 256;
-constexpr int64_t kSelRowPairs = (int64_t)1 << 21;
-static bool sel_row_fits(int conv, int64_t topk, int64_t nblk, int64_t rows, bool mfma) {
-  const int64_t most = conv == FBSA_SEL_OWN_FIRST ? nblk - 1 : nblk, K = topk < most ? topk : most;
-  return nblk <= kSelRowMax && K <= kSelListMax && rows < 0x7fffffffLL && !(mfma && rows * nblk > kSelRowPairs);
+constexpr int64_t kSelRowPairs = (int64_t)1 << 21;  // (row, candidate) pairs up to which the MFMA estimate was fitted
+static bool sel_row_fits(const SelArgs &a, int64_t es, int64_t D, int score, bool mfma) {
+  const bool convA = a.conv == FBSA_SEL_OWN_FIRST;
+  const int64_t most = convA ? a.nblk - 1 : a.nblk, K = a.topk < most ? a.topk : most;
+  const int64_t rows = a.B * a.H * a.nblk;
+  if (a.nblk > kSelRowMax || K > kSelListMax || rows >= 0x7fffffffLL) return false;
+  if (mfma && rows * a.nblk > kSelRowPairs) return false;
+  const double n = (double)a.nblk, set = n * D * (score == FBSA_SCORE_DOT ? 1 : 2);  // elements of a row's candidates
+  const double row = 4 + (K > 32 ? 9 : 0) + 5.2 * rows / (1 << 14) + 26.3 * (rows * set * es) / (1 << 28);
+  if (mfma) {
+    // nearly constant, plus what 512 row blocks of 64 do not cover at once
+    const double rb = (double)(a.B * a.H * ((a.nblk + 63) / 64));
+    return row <= 32 + 0.9 * K + (a.sel_score ? 25 : 0) + (convA ? 0 : 8) + (rb > 512 ? 0.06 * (rb - 512) : 0);
+  }
+  const double wg = (double)(a.B * a.H * ((a.nblk + 7) / 8)) / 1024;  // workgroups of eight rows, in rounds of four a CU
+  const double ins = K > 32 ? n * (5.6 + 13.2 * wg) / 64 : 0;         // candidates inserted one by one
+  return row <= 25 + 27 * wg + 3.4 * n * wg / 64 + ins + set * (0.83 + (9.4 + 2.25 * es) * wg) / (1 << 14);
 }
 
 // Budgets up to 32: past that the pass-1 bound (the K-th of 64 stream maxima)
@@ -1954,7 +1972,7 @@ template <typename T, int D, int MODE> static bool sel_tiled_ok(const SelArgs &a
 template <typename T, int D, int MODE> static int launch_sel(const SelArgs &a, void *ws, hipStream_t s) {
   if (a.row1 <= a.row0) return FBSA_OK;
   const bool mfma = ws && sel_tiled_ok<T, D, MODE>(a);
-  if (!a.chunked && sel_row_fits(a.conv, a.topk, a.nblk, a.B * a.H * a.nblk, mfma)) {
+  if (!a.chunked && sel_row_fits(a, sizeof(T), D, MODE, mfma)) {
     const int64_t nr = a.B * a.H * (a.row1 - a.row0);
     hipLaunchKernelGGL((select_row_kernel<T, D, MODE>), dim3((unsigned)((nr + 3) / 4)), dim3(256), 0, s, a);
     return hip_check(hipGetLastError(), "select_row_kernel launch");
@@ -2068,7 +2086,7 @@ int run_select(const fbsa_select_desc *d, int64_t row0, int64_t row1, const void
 
 // Mean-pooled q.k selection. q and k of dim 32 or 64 are pooled by one launch;
 // where the MFMA engine follows (16-bit operands, its workspace, a budget of at
-// most 32, more blocks than select_row_kernel takes) it also writes the
+// most 32, not select_row_kernel) it also writes the
 // selection's row norms (query side into the first norm array, candidate side
 // into the third; DOT scores use no others). Otherwise pool, pool and select run
 // as three calls. Either way qp, kp and sel are the same.
@@ -2105,8 +2123,10 @@ int run_select_mean_pooled(const fbsa_pool_desc *dq, const void *q, void *qp, co
                            void *kp, const fbsa_select_desc *d, int32_t *sel, float *sel_score, void *ws, hipStream_t s) {
   const int64_t K = d->topk < d->nblk - 1 ? d->topk : d->nblk - 1;
   const bool pair = (d->D == 32 || d->D == 64) && (dq->bs == 16 || dq->bs == 32 || dq->bs == 64 || dq->bs == 128);
+  SelArgs a = {};  // (what sel_row_fits reads: the same choice as launch_sel's)
+  a.conv = d->convention; a.topk = d->topk; a.nblk = d->nblk; a.B = d->B; a.H = d->H; a.sel_score = sel_score;
   const bool norms = pair && ws && d->dtype != FBSA_F32 && K >= 1 && K <= 32 &&
-                     !sel_row_fits(d->convention, d->topk, d->nblk, d->B * d->H * d->nblk, true);
+                     !sel_row_fits(a, 2, d->D, FBSA_SCORE_DOT, true);
   if (!pair) {
     int e = run_pool(dq, q, qp, nullptr, s);
     if (!e) e = run_pool(dk, k, kp, nullptr, s);

@@ -370,6 +370,27 @@ def test_select_tiled_modes(dtype, D, score, conv, causal, topk, ties, chunk):
     assert np.array_equal(sc.cpu().numpy().astype(np.float64), np.take_along_axis(raw, ref, -1))
 
 
+@pytest.mark.parametrize("dtype,D,score,B,nblk,topk", [
+    ("f32", 256, "max2", 32, 256, 8), ("f32", 256, "quest", 8, 256, 8), ("f32", 256, "dot", 32, 256, 8),
+    ("f32", 128, "max2", 32, 256, 8), ("f32", 64, "dot", 64, 256, 8), ("f32", 256, "max2", 64, 256, 62),
+    ("bf16", 64, "max2", 128, 128, 8), ("bf16", 64, "quest", 32, 256, 8), ("bf16", 64, "dot", 512, 64, 8),
+])
+def test_select_row_kernel_is_taken_where_it_is_quicker(dtype, D, score, B, nblk, topk):
+    # a chunk size rules the row kernel out: the choice made without one takes at most 1.3 times
+    # the other engine's time
+    from fbsa_amd import selection
+    g = torch.Generator().manual_seed(47)
+    a, b1, b2 = (randn(g, (B, 1, nblk, D), dtype, device=DEV) for _ in range(3))
+    kw = dict(score=score, topk=topk, causal=True, engine="auto")
+
+    def run(chunk):
+        return lambda: selection.select(a, b1, None if score == "dot" else b2, chunk_tiles=chunk, **kw)
+    assert torch.equal(run(0)(), run(64)())
+    t, other = _us(run(0)), _us(run(64))
+    _say("choice", dtype, D, score, B, nblk, topk, t, other)
+    assert t <= 1.3 * other + 3, (t, other)
+
+
 @pytest.mark.parametrize("dtype,score,conv,causal,topk,nblk,ties", [
     ("bf16", "dot", "own_first", True, 64, 900, False),
     ("bf16", "dot", "own_first", True, 128, 900, True),
