@@ -175,6 +175,17 @@ def test_select_mean_pooled_exact(dtype, B, H, N, bs, topk, causal, engine):
     ("bf16", 1, 2, 2, 4096, 32, 64, 16, 1e-20),    # norms below 2^-40: likewise
     ("bf16", 3, 1, 1, 3000, 64, 32, 16, 1.0),      # one head: plain token means, a block per wave
     ("f16", 1, 1, 1, 4000, 32, 128, 8, 1.0),
+    # the shapes above have at most 256 blocks and run select_row_kernel; past that the pooling
+    # writes the row norms that the MFMA engine starts from
+    ("bf16", 1, 8, 8, 16448, 64, 64, 16, 1.0),     # 257 blocks
+    ("bf16", 2, 4, 2, 9000, 64, 32, 32, 1.0),      # ragged tail block, largest fused budget
+    ("bf16", 2, 4, 2, 9000, 64, 32, 33, 1.0),      # past it: no norms, fp64 select
+    ("f16", 1, 2, 1, 8192, 32, 16, 8, 1.0),
+    ("bf16", 1, 2, 2, 8192, 64, 16, 16, 1e19),     # norms past 1e18
+    ("bf16", 1, 2, 2, 8192, 32, 16, 16, 1e-20),    # norms below 2^-40
+    ("bf16", 3, 1, 1, 9000, 64, 32, 16, 1.0),      # one head: plain token means
+    ("f16", 1, 1, 1, 8192, 32, 16, 8, 1.0),
+    ("bf16", 40, 2, 1, 4096, 64, 16, 16, 1.0),     # 256 blocks, but more pairs than the row kernel takes
 ])
 def test_select_mean_pooled_fused_equals_separate_calls(dtype, B, Hq, Hk, N, D, bs, topk, scale):
     """fbsa_select_mean_pooled (q and k pooled by one launch that also writes the
@@ -370,6 +381,24 @@ def test_select_tiled_modes(dtype, D, score, conv, causal, topk, ties, chunk):
     assert np.array_equal(sc.cpu().numpy().astype(np.float64), np.take_along_axis(raw, ref, -1))
 
 
+@pytest.mark.parametrize("B,nblk,scale", [(1, 300, 1e19), (1, 300, 1e-20), (33, 256, 1.0), (33, 256, 1e19)])
+@pytest.mark.parametrize("D", [32, 64])
+def test_select_mfma_engine_equals_fp64(B, nblk, scale, D):
+    # past 256 blocks, or with more than 2^21 (row, candidate) pairs, "auto" is the MFMA engine
+    # with its exact check of ambiguous pairs (every pair where the norms are past 1e18 or below
+    # 2^-40); sampled rows against the oracle as well
+    from fbsa_amd import selection
+    g = torch.Generator().manual_seed(41)
+    a, b = ((torch.randn(B, 1, nblk, D, generator=g) * scale).to(torch.bfloat16) for _ in range(2))
+    _say("mfma against fp64", B, nblk, scale, D)
+    kw = dict(topk=16, causal=True, need_scores=True)
+    sel1, sc1 = selection.select(a.to(DEV), b.to(DEV), engine="auto", **kw)
+    sel2, sc2 = selection.select(a.to(DEV), b.to(DEV), engine="fp64", **kw)
+    assert torch.equal(sel1, sel2) and torch.equal(sc1, sc2)
+    raw = osel.scores(np64(a[:1]), np64(b[:1]), "bf16", "dot")
+    _check_sel(sel1[:1, 0].cpu().numpy(), osel.select_conv_a(raw[:, 0], 16, True), "sel")
+
+
 @pytest.mark.parametrize("dtype,D,score,B,nblk,topk", [
     ("f32", 256, "max2", 32, 256, 8), ("f32", 256, "quest", 8, 256, 8), ("f32", 256, "dot", 32, 256, 8),
     ("f32", 128, "max2", 32, 256, 8), ("f32", 64, "dot", 64, 256, 8), ("f32", 256, "max2", 64, 256, 62),
@@ -389,6 +418,64 @@ def test_select_row_kernel_is_taken_where_it_is_quicker(dtype, D, score, B, nblk
     t, other = _us(run(0)), _us(run(64))
     _say("choice", dtype, D, score, B, nblk, topk, t, other)
     assert t <= 1.3 * other + 3, (t, other)
+
+
+@pytest.mark.parametrize("engine", ["auto", "fp64"])
+@pytest.mark.parametrize("nblk", [1, 2, 63, 64, 65, 128, 129, 255, 256])
+@pytest.mark.parametrize("dtype,D,score,conv,causal,topk,kind", [
+    ("bf16", 64, "dot", "own_first", True, 16, "ties"), ("bf16", 32, "dot", "own_first", False, 62, "ties"),
+    ("f16", 16, "max2", "own_first", True, 5, "ties"), ("f32", 64, "dot", "own_first", True, 8, "plain"),
+    ("f32", 256, "quest", "sorted_sink", True, 30, "ties"), ("bf16", 128, "quest", "sorted_sink", True, 62, "plain"),
+    ("f16", 64, "dot", "own_first", True, 16, "special"), ("bf16", 32, "dot", "sorted_sink", True, 62, "special"),
+    ("f32", 32, "dot", "own_first", False, 7, "special"), ("bf16", 64, "quest", "sorted_sink", True, 16, "special"),
+    ("bf16", 64, "dot", "own_first", True, 0, "plain"),
+])
+def test_select_row_kernel(dtype, D, score, conv, causal, topk, kind, nblk, engine):
+    # one wave per row (up to 256 blocks, budgets up to 62): exact ties, NaN and infinite scores
+    # on both sides of the 64th candidate, where ranking by lane reads ends and inserting begins
+    from fbsa_amd import selection
+    g = torch.Generator().manual_seed(nblk + D)
+    B, H = 2, 2
+    if kind == "ties":
+        dt = randn(g, (1,), dtype).dtype
+        mk = lambda: torch.randint(-1, 2, (B, H, nblk, D), generator=g).to(dt)  # noqa: E731
+    else:
+        mk = lambda: randn(g, (B, H, nblk, D), dtype)  # noqa: E731
+    a, b1, b2 = mk(), mk(), mk()
+    if score == "quest":
+        b1, b2 = torch.maximum(b1, b2), torch.minimum(b1, b2)
+    if kind == "special":
+        for j, v in ((0, "nan"), (1, "inf"), (62, "nan"), (63, "inf"), (64, "nan"), (65, "-inf"), (66, "inf"), (200, "nan")):
+            if j < nblk:
+                b1[:, :, j, 3] = float(v)
+    _say("row kernel", dtype, D, score, conv, causal, topk, kind, nblk, engine)
+    sel, sc = selection.select(a.to(DEV), b1.to(DEV), None if score == "dot" else b2.to(DEV), score=score, convention=conv,
+                               topk=topk, causal=causal, sink=conv == "sorted_sink", need_scores=True, engine=engine)
+    with np.errstate(invalid="ignore", over="ignore"):
+        raw = osel.scores(np64(a), np64(b1), dtype, score, b2=None if score == "dot" else np64(b2))
+    if conv == "own_first":
+        ref = np.stack([osel.select_conv_a(raw[:, h], topk, causal) for h in range(H)], 1)
+    else:
+        ref = osel.select_conv_b(raw, topk, True)
+    _check_sel(sel.cpu().numpy(), ref, "sel")
+    # (a slot that repeats the own block in place of a non-finite pick carries its score)
+    assert np.array_equal(sc.cpu().numpy().astype(np.float64), np.take_along_axis(raw, ref, -1), equal_nan=True)
+
+
+@pytest.mark.parametrize("r0,r1", [(1, 2), (37, 101), (64, 130), (129, 130)])
+def test_select_row_kernel_row_range(r0, r1):
+    from fbsa_amd import selection
+    g = torch.Generator().manual_seed(43)
+    B, H, nblk, D, topk = 2, 2, 130, 64, 9
+    a, b = (randn(g, (B, H, nblk, D), "bf16") for _ in range(2))
+    out = torch.full((B, H, nblk, topk + 1), -7, dtype=torch.int32, device=DEV)
+    _say("row kernel rows", r0, r1)
+    selection.select(a.to(DEV), b.to(DEV), topk=topk, causal=True, rows=(r0, r1), out=out)
+    raw = osel.scores(np64(a), np64(b), "bf16", "dot")
+    ref = np.full(out.shape, -7)
+    for h in range(H):
+        ref[:, h, r0:r1] = osel.select_conv_a(raw[:, h], topk, True)[:, r0:r1]
+    _check_sel(out.cpu().numpy(), ref, "sel")
 
 
 @pytest.mark.parametrize("dtype,score,conv,causal,topk,nblk,ties", [
