@@ -193,6 +193,14 @@ int fbsa_block_mass(const fbsa_attn_desc *d, const void *q, const void *k, float
   return run_block_mass(d, q, k, mass, ws, (hipStream_t)stream);
 }
 
+int fbsa_block_mass_sized(const fbsa_attn_desc *d, const void *q, const void *k, float *mass, void *ws,
+                          size_t workspace_bytes, void *stream) {
+  const size_t need = fbsa_block_mass_workspace_bytes(d);
+  if (ws && workspace_bytes < need)
+    return fail(FBSA_EWORKSPACE, "fbsa_block_mass: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+  return fbsa_block_mass(d, q, k, mass, ws, stream);
+}
+
 static int check_pool(const fbsa_pool_desc *d, const void *x, const void *out, const void *out2) {
   if (!d) return fail(FBSA_EINVAL, "fbsa_pool: null descriptor");
   if (d->dtype < FBSA_F32 || d->dtype > FBSA_F16) return fail(FBSA_EINVAL, "fbsa_pool: bad dtype %d", d->dtype);

@@ -80,6 +80,7 @@ SIGNATURES = {
                       + [_vp] * 9),
     "fbsa_block_mass_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnDesc)]),
     "fbsa_block_mass": (ctypes.c_int, [ctypes.POINTER(AttnDesc), _vp, _vp, _vp, _vp, _vp]),
+    "fbsa_block_mass_sized": (ctypes.c_int, [ctypes.POINTER(AttnDesc), _vp, _vp, _vp, _vp, ctypes.c_size_t, _vp]),
     "fbsa_pool": (ctypes.c_int, [ctypes.POINTER(PoolDesc), _vp, _vp, _vp, _vp]),
     "fbsa_select_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(SelectDesc)]),
     "fbsa_select": (ctypes.c_int, [ctypes.POINTER(SelectDesc), _vp, _vp, _vp, _vp, _vp, _vp,

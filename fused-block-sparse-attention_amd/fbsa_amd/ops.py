@@ -280,7 +280,9 @@ def block_mass(q, k, bs, scale=None):
     d.sk[:] = _strides3(qk[1])
     lib = _lib.load()
     mass = torch.empty(B, Hq, nblk, nblk, dtype=torch.float32, device=q.device)
-    ws = torch.empty((lib.fbsa_block_mass_workspace_bytes(d) + 3) // 4, dtype=torch.float32, device=q.device)
-    _lib.check(lib.fbsa_block_mass(d, _ptr(qk[0]), _ptr(qk[1]), _ptr(mass), _ptr(ws), _stream()), "fbsa_block_mass")
+    nbytes = lib.fbsa_block_mass_workspace_bytes(d)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+    _lib.check(lib.fbsa_block_mass_sized(d, _ptr(qk[0]), _ptr(qk[1]), _ptr(mass), _ptr(ws), nbytes, _stream()),
+               "fbsa_block_mass")
     return mass
 

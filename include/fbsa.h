@@ -99,9 +99,15 @@ int fbsa_fwd_rows(const fbsa_attn_desc *d, int64_t i_begin, int64_t i_end, const
  * rnd(rnd(q.k) * scale); the softmax is fp32. Reads d->dtype (bf16 or f16),
  * B, Hq, Hkv, L = nblk * bs, D (64, 128, 256), bs (64, 128), nblk, scale, sq,
  * sk. ws: fbsa_block_mass_workspace_bytes(d) bytes, 16-byte aligned (each
- * row's unnormalised sums per key block; at most 1 GiB or 256 query blocks'
- * worth, longer sequences run in several launches). Replaces the per-query-block loop of capture_mass. */
+ * row's unnormalised sums per key block, 6 bytes per (row, key block); at most
+ * 1 GiB or 256 query blocks' worth, whichever is more; longer sequences run in
+ * several launches). The size grows with the square of L and is not the B*Hq*L
+ * floats that the row log-sum-exp alone would take: fbsa_block_mass is given no
+ * size and writes that much, fbsa_block_mass_sized refuses a workspace_bytes
+ * below it (FBSA_EWORKSPACE). Replaces the per-query-block loop of capture_mass. */
 size_t fbsa_block_mass_workspace_bytes(const fbsa_attn_desc *d);
+int fbsa_block_mass_sized(const fbsa_attn_desc *d, const void *q, const void *k, float *mass, void *ws,
+                          size_t workspace_bytes, void *stream);
 int fbsa_block_mass(const fbsa_attn_desc *d, const void *q, const void *k, float *mass, void *ws, void *stream);
 
 /* ---- selection ------------------------------------------------------- */

@@ -77,6 +77,23 @@ def test_fwd_rejects_null_and_misaligned_pointers():
     assert lib.fbsa_fwd(d, DUMMY, DUMMY, DUMMY, DUMMY, None, None, DUMMY, None, None) == _lib.EINVAL
 
 
+def test_block_mass_checks_its_workspace():
+    lib = _lib.load()
+    d = _desc(mask=_lib.MASK_TOKEN_CAUSAL, kk=1)
+    need = lib.fbsa_block_mass_workspace_bytes(d)
+    assert need == 2 * 4 * 256 * 6                # every (head, query block): a sum and a score per (row, key block)
+    for short in (0, 2 * 256 * 4, need - 1):      # (the row log-sum-exp alone is B * Hq * L floats)
+        assert lib.fbsa_block_mass_sized(d, DUMMY, DUMMY, DUMMY, DUMMY, short, None) == _lib.EWORKSPACE
+        assert "workspace" in lib.fbsa_last_error().decode()
+    assert lib.fbsa_block_mass_sized(d, DUMMY, DUMMY, DUMMY, None, 0, None) == _lib.EINVAL
+    assert lib.fbsa_block_mass_sized(None, DUMMY, DUMMY, DUMMY, DUMMY, 0, None) == _lib.EINVAL
+    # past the cap: 256 workgroups of the longest walk when that is more than 1 GiB
+    n = 1 << 20
+    d.L = d.l_valid = n
+    d.nblk = n // 64
+    assert lib.fbsa_block_mass_workspace_bytes(d) == 256 * n * 6 > 1 << 30
+
+
 def test_select_rejects_bad_budget():
     lib = _lib.load()
     d = _lib.SelectDesc()
