@@ -837,9 +837,9 @@ __global__ __launch_bounds__(BS * 4, (dq_minwg<T, BS, D>())) void dq_kernel(BwdA
   TilePairPlan<T, C::KC, D, C::NW, C::LPT> plan;
   plan.init(a.sk[2], a.sv[2], w, lane);
   // list entries read an iteration ahead, as in the forward (with that the asm
-  // copies are the faster form at every head dim: 262144 tokens, d 64, dQ within
-  // a training step 4.01 -> 3.98 ms against copies through the builtin, which
-  // had been faster while each issue waited for its list read)
+  // copies are the faster form at d 64 too, 32 x 1024-token training step 330 ->
+  // 325 us, or no slower, 262144 tokens within what runs differ; copies through the
+  // builtin had been faster while each issue waited for its list read)
   int islot = 0, ich = 0, ist = 0;  // chunk to issue next: slot, place in the slot, stage
   int slot = 0, ch = 0, cst = 0;    // chunk to compute next
   int f_iblk, f_kind;
