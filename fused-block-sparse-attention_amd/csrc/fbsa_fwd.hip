@@ -224,18 +224,27 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
   // of the one before: they land by the barrier, go to scalar registers there,
   // and neither the issue nor the softmax waits for an LDS read (65536 tokens, d
   // 256, 34 slots: 0.8%, runs differing by 0.3%; d 64, one chunk per slot: unchanged).
+  // A dense walk has no list: with several chunks to a block their places come from
+  // the chunk's number, and the mask kind is formed beside the products. Reading
+  // ahead put that work between the barrier and the issue, 4 to 6% at blocks of 128
+  // (4096 tokens, 8 heads, d 64: 162 -> 153 us; 8192 tokens, 16 heads over 2, d 256:
+  // 608 -> 584). With one chunk to a block the stepped places are 2 to 4% ahead.
+  constexpr bool AHEAD = !DENSE || C::NCH == 1;
   int islot = 0, ich = 0, ist = 0;  // chunk to issue next: slot, place in the slot, stage
   int slot = 0, ch = 0, cst = 0;    // chunk to compute next
   int f_iblk, f_kind;
   float f_gate;
   auto fetch = [&]() {  // (past the end: the last entry again, unused; without one, place 0's stale bytes)
+    if constexpr (!AHEAD) return;
     const int last = nv > 0 ? nv - 1 : 0, si = islot < last ? islot : last, sc = slot < last ? slot : last;
     f_iblk = blk_of(si);
     f_kind = kind_of(sc);
     f_gate = DENSE ? 0.f : s_gate[sc];
   };
-  auto issue = [&]() {
-    const uint32_t first = (uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC);
+  auto issue = [&](int c) {
+    if constexpr (!AHEAD) ist = c % C::NSTAGE;
+    const uint32_t first = AHEAD ? (uint32_t)(__builtin_amdgcn_readfirstlane(f_iblk) * BS + ich * C::KC)
+                                 : (uint32_t)(c * C::KC);
     const uint32_t row0 = RAGGED ? tail_row(first, (uint32_t)a.rows) : first;
     const char *kb = kbase + (int64_t)row0 * kstep, *vb = vbase + (int64_t)row0 * vstep;
     const uint32_t kl = tail_limit<C::KC>(row0, (uint32_t)a.rows, (uint32_t)kstep, D * C::ES);
@@ -247,8 +256,10 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
       const uint32_t lim = part ? vl : kl, off = (uint32_t)doff[n];
       g2lds16_s(part ? vb : kb, RAGGED && off > lim ? lim : off, st + (n * C::NW + w) * 1024);
     }
-    ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
-    if (++ich == C::NCH) { ich = 0; ++islot; }
+    if constexpr (AHEAD) {
+      ist = ist + 1 == C::NSTAGE ? 0 : ist + 1;
+      if (++ich == C::NCH) { ich = 0; ++islot; }
+    }
   };
 
   // Online softmax in the log2 domain with a lazily moved reference max: the
@@ -273,7 +284,7 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
   for (int c = 0; c < C::NSTAGE - 1; ++c)
     if (c < nchunks) {
       fetch();
-      issue();
+      issue(c);
     }
   fetch();
   // the register-operand loads above and the first stages have landed (issued
@@ -298,10 +309,19 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
     // one barrier per chunk: every wave has landed its part of chunk c and
     // finished reading chunk c-1, whose stage the prefetch below overwrites
     lds_barrier();
-    const int kind = __builtin_amdgcn_readfirstlane(f_kind);
-    const float gt = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f_gate)));
+    int kind = 0;
+    float gt = 0.f;
+    if constexpr (AHEAD) {
+      kind = __builtin_amdgcn_readfirstlane(f_kind);
+      gt = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(f_gate)));
+    } else {
+      slot = c / C::NCH;
+      ch = c % C::NCH;
+      cst = c % C::NSTAGE;
+    }
     const int cslot = slot, cch = ch;
-    if (c + C::NSTAGE - 1 < nchunks) issue();
+    if (c + C::NSTAGE - 1 < nchunks) issue(c + C::NSTAGE - 1);
+    if constexpr (!AHEAD) kind = kind_of(slot);  // (scalar work beside the products)
 
     const char *Ks = stages + cst * C::STAGE_BYTES;
     const char *Vs = Ks + C::TILE_BYTES;
@@ -490,8 +510,10 @@ __global__ __launch_bounds__(BS * 4 / QT) void fwd_kernel(FwdArgs a) {
         }
       }
     }
-    cst = cst + 1 == C::NSTAGE ? 0 : cst + 1;
-    if (++ch == C::NCH) { ch = 0; ++slot; }
+    if constexpr (AHEAD) {
+      cst = cst + 1 == C::NSTAGE ? 0 : cst + 1;
+      if (++ch == C::NCH) { ch = 0; ++slot; }
+    }
     fetch();
   }
 
